@@ -1127,6 +1127,150 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
     write_tile<BM, BN, WGM, WGN, RING, EP>(p, acc, smem, m0, n0, tn);
 }
 
+// INT8 GEMM for outputs with too few 256 x 256 tiles to fill the chip (Dequant or Int32 epilogue): a BM x BN x
+// 128 tile of four waves (one per SIMD), each a (BM / 2) x (BN / 2) block of v_mfma_i32_32x32x32_i8
+// accumulators.  The integer sums are exact, so the results are those of every other GEMM kernel here bit for
+// bit.
+//
+// What bounds a lone tile is the operand stream of its CU, not the matrix pipe: LDS-DMA alone (no MFMA, no
+// fragment reads) takes 0.37 us per 32 KB K step of a 128 x 128 tile, its MFMAs 0.21 us, and a DMA
+// instruction holds up the wave that issues it, so with the loads issued ahead of the MFMAs the two added up
+// (0.52 us).  Here a wave holds all fragments of a K step in registers (two buffers), and under the MFMAs of
+// step k it reads the fragments of step k + 1 (first half of the MFMAs) and issues its share of the DMA of
+// step k + NS (second half): 0.43 us per step on 64 CUs, 0.57 us on 240.  The reads come first in program
+// order because LDS-DMA writes the same LDS and the compiler keeps them in order.
+//
+// Ring of NS stages, one barrier per K step: it publishes stage k + 1 (each wave has waited for its own loads)
+// and frees the slot of stage k, whose fragments every wave has in registers by then.
+template <int BM, int BN, int NS, Epi EP>
+__global__ __launch_bounds__(256) void gemm_i8_small(GemmParams p) {
+    static_assert(EP == Epi::Dequant || EP == Epi::Int32, "decoder GEMM epilogues");
+    constexpr int BK = 128, NW = 4, WGM = 2, WGN = 2;
+    constexpr int WM = BM / WGM, WN = BN / WGN, FM = WM / 32, FN = WN / 32, KS = BK / 32;
+    constexpr int A_BYTES = BM * BK, STAGE = (BM + BN) * BK, RING = NS * STAGE;
+    constexpr int A_PW = BM / 8 / NW, B_PW = BN / 8 / NW, LPS = A_PW + B_PW;   // DMA instructions per wave and stage
+    static_assert(A_PW * 8 * NW == BM && B_PW * 8 * NW == BN, "tile rows must split into eight-row groups per wave");
+    static_assert(NS >= 2 && NS * LPS < 64 && RING <= 163840, "ring");
+
+    extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar)
+    const int wm = wave / WGN, wn = wave % WGN;
+    int tm, tn;
+    grouped_tile(xcd_remap(blockIdx.x, gridDim.x), p.tiles_m, p.tiles_n, 8, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int nk = p.K / BK;
+
+    // DMA: eight rows of 128 bytes per instruction, as in gemm_i8_pingpong
+    const int lrow = lane >> 3, lslot = lane & 7;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)p.a_bytes, kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, (int)p.b_bytes, kRsrcWord3);
+    uint32_t aoff[A_PW], boff[B_PW];
+#pragma unroll
+    for (int j = 0; j < A_PW; ++j) {
+        const int r = (wave * A_PW + j) * 8 + lrow;
+        const int m = m0 + r < p.M ? m0 + r : p.M - 1;
+        aoff[j] = (uint32_t)((int64_t)m * p.lda + ((lslot ^ swz<BK>(r)) << 4));
+    }
+#pragma unroll
+    for (int j = 0; j < B_PW; ++j) {
+        const int r = (wave * B_PW + j) * 8 + lrow;
+        const int n = n0 + r < p.N ? n0 + r : p.N - 1;
+        boff[j] = (uint32_t)((int64_t)n * p.K + ((lslot ^ swz<BK>(r)) << 4));
+    }
+    auto issue = [&](int k, int slot) {
+        int8_t* sa = smem + slot * STAGE;
+#pragma unroll
+        for (int j = 0; j < B_PW; ++j) lds_dma16(rb, boff[j], (uint32_t)(k * BK), sa + A_BYTES + (wave * B_PW + j) * 1024);
+#pragma unroll
+        for (int j = 0; j < A_PW; ++j) lds_dma16(ra, aoff[j], (uint32_t)(k * BK), sa + (wave * A_PW + j) * 1024);
+    };
+
+    const int frow = lane & 31, fhi = lane >> 5;
+    v4i fa[2][KS][FM], fb[2][KS][FN];
+    auto load_frags = [&](int slot, auto buf) {
+        constexpr int B = decltype(buf)::value;
+        const int8_t* sa = smem + slot * STAGE;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int kc = fhi + 2 * ks;
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                const int r = wm * WM + i * 32 + frow;
+                fa[B][ks][i] = *reinterpret_cast<const v4i*>(sa + r * BK + ((kc ^ swz<BK>(r)) << 4));
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int r = wn * WN + j * 32 + frow;
+                fb[B][ks][j] = *reinterpret_cast<const v4i*>(sa + A_BYTES + r * BK + ((kc ^ swz<BK>(r)) << 4));
+            }
+        }
+    };
+
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+        if (s < nk) issue(s, s);
+    v16i acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = v16i{};
+    if (nk >= NS) wait_vmcnt<(NS - 1) * LPS>();
+    else wait_vmcnt<0>();
+    lds_barrier();
+    load_frags(0, std::integral_constant<int, 0>{});
+
+    int slot = 0;
+    // K step k on fragment buffer B.  FULL: a stage k + NS follows (its DMA then sits in the same basic block as
+    // the MFMAs and is spread over them).
+    auto step = [&](int k, auto buf, auto full) {
+        constexpr int B = decltype(buf)::value;
+        constexpr bool FULL = decltype(full)::value;
+        const int nslot = slot + 1 == NS ? 0 : slot + 1;
+        // stage k + 1 landed; stages k + 2 .. k + NS - 1 may be in flight
+        if (FULL || k + NS <= nk) wait_vmcnt<(NS - 2) * LPS>();
+        else wait_vmcnt<0>();
+        lds_barrier();
+        if (!FULL && k + NS < nk) issue(k + NS, slot);
+        __builtin_amdgcn_sched_barrier(0);
+        load_frags(nslot, std::integral_constant<int, B ^ 1>{});   // after the last step a stale slot, never used
+        if constexpr (FULL) issue(k + NS, slot);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[B][ks][j], fa[B][ks][i], acc[i][j], 0, 0, 0);
+        constexpr int NM = KS * FM * FN, NR = KS * (FM + FN), H = NM / 2;
+        constexpr int RP = FULL ? (NR + H - 1) / H : (NR + NM - 1) / NM, DP = (LPS + H - 1) / H;
+#pragma unroll
+        for (int g = 0; g < NM; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (!FULL || g < H) __builtin_amdgcn_sched_group_barrier(0x100, RP, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x010, DP, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        slot = nslot;
+    };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    int k = 0;
+    for (; k + 1 + NS < nk; k += 2) {
+        step(k, B0{}, std::true_type{});
+        step(k + 1, B1{}, std::true_type{});
+    }
+    for (; k + 1 < nk; k += 2) {
+        step(k, B0{}, std::false_type{});
+        step(k + 1, B1{}, std::false_type{});
+    }
+    if (k < nk) step(k, B0{}, std::false_type{});
+
+    write_tile<BM, BN, WGM, WGN, RING, EP>(p, acc, smem, m0, n0, tn);
+}
+
 // Ping-pong INT8 GEMM (AMode::Gemm, Dequant or Int32 epilogue): 256 x 256 x 128 tiles, 8 waves in two
 // groups of four (one wave of each group per SIMD: wave w runs on SIMD w % 4).  Group g owns output rows
 // 128 g .. 128 g + 127 of the tile, and wave s of a group the 64 columns 64 s .. 64 s + 63: a 128 x 64 block
@@ -2050,28 +2194,50 @@ int launch_halo(GemmParams p, hipStream_t stream, const char* what) {
     return launch_status(what);
 }
 
-template <Epi EP>
-int launch_pingpong(GemmParams p, hipStream_t stream, const char* what) {
-    p.tiles_m = (p.M + 255) / 256;
-    p.tiles_n = (p.N + 255) / 256;
+// Tile counts, epilogue forms and operand extents of a K % 128 == 0 GEMM on BM x BN tiles.
+template <int BM, int BN>
+int fill_gemm_tiles(GemmParams& p, const char* what) {
+    p.tiles_m = (p.M + BM - 1) / BM;
+    p.tiles_n = (p.N + BN - 1) / BN;
     p.vec_epi = (p.sw == nullptr || aligned(p.sw, 16)) && (p.bias == nullptr || aligned(p.bias, 8)) && p.N % 4 == 0;
     p.vec_out = aligned(p.out, 16) && p.ldo % 8 == 0;
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    if (tiles > 0x7fffffff) return fail(H3V_EINVAL, "%s: too many tiles", what);
+    if ((int64_t)p.tiles_m * p.tiles_n > 0x7fffffff) return fail(H3V_EINVAL, "%s: too many tiles", what);
     const int64_t a_bytes = (int64_t)p.M * p.lda, b_bytes = (int64_t)p.N * p.K;
     if (a_bytes >= ((int64_t)1 << 32) || b_bytes >= ((int64_t)1 << 32))
         return fail(H3V_EINVAL, "%s: an operand exceeds 4 GiB (%lld, %lld bytes)", what, (long long)a_bytes,
                     (long long)b_bytes);
     p.a_bytes = (uint32_t)a_bytes;
     p.b_bytes = (uint32_t)b_bytes;
-    constexpr size_t lds = 5 * 256 * 128;   // three activation and two weight slots: 160 KB
-    auto kernel = &gemm_i8_pingpong<EP>;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return H3V_OK;
+}
+
+int launch_gemm_tiles(const void* kernel, hipError_t attr, size_t lds, int threads, const GemmParams& p,
+                      hipStream_t stream, const char* what) {
     if (attr != hipSuccess) return fail(H3V_ELAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", what, lds,
                                         hipGetErrorString(attr));
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(512), lds, stream, p);
+    hipLaunchKernelGGL(reinterpret_cast<void (*)(GemmParams)>(const_cast<void*>(kernel)),
+                       dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3((unsigned)threads), lds, stream, p);
     return launch_status(what);
+}
+
+template <Epi EP>
+int launch_pingpong(GemmParams p, hipStream_t stream, const char* what) {
+    const int rc = fill_gemm_tiles<256, 256>(p, what);
+    if (rc) return rc;
+    constexpr size_t lds = 5 * 256 * 128;   // three activation and two weight slots: 160 KB
+    const void* kernel = reinterpret_cast<const void*>(&gemm_i8_pingpong<EP>);
+    static const hipError_t attr = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return launch_gemm_tiles(kernel, attr, lds, 512, p, stream, what);
+}
+
+template <int BM, int BN, int NS, Epi EP>
+int launch_small(GemmParams p, hipStream_t stream, const char* what) {
+    const int rc = fill_gemm_tiles<BM, BN>(p, what);
+    if (rc) return rc;
+    constexpr size_t lds = (size_t)NS * (BM + BN) * 128;
+    const void* kernel = reinterpret_cast<const void*>(&gemm_i8_small<BM, BN, NS, EP>);
+    static const hipError_t attr = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return launch_gemm_tiles(kernel, attr, lds, 256, p, stream, what);
 }
 
 template <AMode AM, Epi EP>
@@ -2083,6 +2249,61 @@ int launch_generic(GemmParams p, hipStream_t stream, const char* what) {
     return launch_status(what);
 }
 
+enum class SmallTile { None, T64, T128, T128x2 };
+
+// Tile of gemm_i8_small for an M x N output, None when the 256 x 256 ping-pong tiles are faster.  Measured over
+// M 64 ... 16384 at the decoder's (K, N) of widths 1024 and 2048 (us, 64 / 128 / 128 with two per CU / ping-pong):
+//   up to 512 tiles of 64 x 64 (two fit a CU)   453 x 2048 x 8192: 16.5 / 27.6 / 45.4 / 67.8;
+//                                               1013 x 2048 x 2048: 9.6 / 11.7 / 15.0 / 22.9;
+//                                               453 x 6144 x 2048 (768 tiles): 14.1 / 12.2 / 15.7 / 23.6;
+//   then up to 256 tiles of 128 x 128           1797 x 2048 x 8192: 49.9 / 35.6 / 50.4 / 69.8;
+//   then up to 512 with a two-stage ring, so    3594 x 2048 x 8192: 96.5 / 68.5 / 62.8 / 76.1;
+//   that two workgroups share a CU              453 x 16384 x 2048: 32.6 / 27.5 / 22.4 / 27.2;
+//   beyond                                      4100 x 2048 x 2048: 35.1 / 36.2 / 33.0 / 28.0.
+SmallTile small_tile(int64_t m, int64_t n) {
+    auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+    if (tiles(64) <= 512) return SmallTile::T64;
+    if (tiles(128) <= 256) return SmallTile::T128;
+    if (tiles(128) <= 512) return SmallTile::T128x2;
+    return SmallTile::None;
+}
+
+template <Epi EP>
+int launch_small_tile(SmallTile t, const GemmParams& p, hipStream_t stream, const char* what) {
+    if (t == SmallTile::T64) return launch_small<64, 64, 4, EP>(p, stream, what);
+    if (t == SmallTile::T128) return launch_small<128, 128, 4, EP>(p, stream, what);
+    return launch_small<128, 128, 2, EP>(p, stream, what);
+}
+
+// Aligned GEMM with K a multiple of 128.  A last round of ping-pong tiles that leaves most CUs idle costs about as
+// much as a full one, so when the rows past the last full round are few enough for the small tiles they run there,
+// as a second launch on the remaining rows: 8405 x 2048 x 8192 (264 ping-pong tiles) 171.8 -> 128.3 us, 8405 x
+// 2048 x 2048 55.0 -> 44.4, 3000 x 6144 x 2048 54.7 -> 47.6, 7188 x 16384 x 2048 (7.25 rounds) 250.4 -> 242.4.
+// After three rounds the tiles' ends are spread out and a larger rest overlaps them (8405 x 16384 x 2048, 256
+// tiles of 128 x 128 left after 8 rounds: 288.6 against 301.0 us split), so there only the 64 x 64 tiles split off.
+template <Epi EP>
+int run_gemm_k128(const GemmParams& p, hipStream_t stream, const char* what) {
+    const SmallTile whole = small_tile(p.M, p.N);
+    if (whole != SmallTile::None) return launch_small_tile<EP>(whole, p, stream, what);
+    const int64_t tn = (p.N + 255) / 256, tiles = (p.M + 255) / 256 * tn;
+    const int64_t head = 256 * (tiles / 256 * 256 / tn);   // rows of the full rounds
+    const bool in_range = (int64_t)p.M * p.lda < ((int64_t)1 << 32) && (int64_t)p.N * p.K < ((int64_t)1 << 32);
+    if (head > 0 && head < p.M && in_range) {
+        const SmallTile rest = small_tile(p.M - head, p.N);
+        if (rest == SmallTile::T64 || (rest != SmallTile::None && tiles < 3 * 256)) {
+            GemmParams h = p, t = p;
+            h.M = (int)head;
+            t.M = (int)(p.M - head);
+            t.a = p.a + head * p.lda;
+            if (p.sx) t.sx = p.sx + head * p.sx_stride;
+            t.out = static_cast<char*>(p.out) + head * p.ldo * (EP == Epi::Int32 ? 4 : 2);
+            const int rc = launch_pingpong<EP>(h, stream, what);
+            return rc ? rc : launch_small_tile<EP>(rest, t, stream, what);
+        }
+    }
+    return launch_pingpong<EP>(p, stream, what);
+}
+
 template <Epi EP>
 int run_gemm(GemmParams p, hipStream_t stream, const char* what) {
     const bool al = p.lda % 16 == 0 && aligned(p.a, 16) && aligned(p.b, 16);
@@ -2090,7 +2311,7 @@ int run_gemm(GemmParams p, hipStream_t stream, const char* what) {
     // than three A stages (FFN-up 7188 x 16384 x 2048: 285 vs 305 us); long K keeps the
     // deeper A ring (FFN-down 7188 x 2048 x 8192: 116 vs 132 us).
     if constexpr (EP == Epi::Dequant || EP == Epi::Int32)
-        if (al && p.K % 128 == 0) return launch_pingpong<EP>(p, stream, what);
+        if (al && p.K % 128 == 0) return run_gemm_k128<EP>(p, stream, what);
     if (al && p.K % 128 == 0 && p.K <= 4096) return launch_tiled<256, 256, 128, 2, 4, 2, 2, AMode::Gemm, EP>(p, stream, what);
     if (al && p.K % 128 == 0) return launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Gemm, EP>(p, stream, what);
     if (al && p.K % 64 == 0) return launch_tiled<256, 256, 64, 2, 4, 4, 4, AMode::Gemm, EP>(p, stream, what);
