@@ -11,7 +11,8 @@
 // slice of the QKV projection and q, k the QK-RoPE outputs, with no copies.
 //
 // One workgroup = 8 waves = 512 queries of one (batch, head); each wave owns
-// two sets of 32 queries.  Keys and values stream in blocks of 64 through LDS:
+// two sets of 32 queries (one set, or 4 waves, where that fills the chip better,
+// see plan_attention).  Keys and values stream in blocks of 64 through LDS:
 //
 //   S = K . Q^T   v_mfma_f32_32x32x16_f16, A = K rows from LDS, B = the wave's
 //                 Q fragments (registers, loaded once).  In the 32 x 32 result
@@ -45,10 +46,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kD = 64;        // head dim
 constexpr int kBK = 64;       // keys per block
-// 32-query sets per wave: two share every K / V^T fragment read (246 VGPRs, 2 waves per SIMD);
-// one set (152 VGPRs, 3 waves per SIMD) measured 5% slower on the H3 shape, 11% on [1, 16384, 16, 64]
-constexpr int kQuerySets = 2;
-constexpr int kThreads = 256;   // the K / V loading threads (waves 0-3); a workgroup has 8 waves
+constexpr int kThreads = 256;   // the K / V loading threads (waves 0-3 of a workgroup)
 constexpr float kLazy = 8.0f;   // log2 margin of the lazy softmax maximum (weights stay <= 2^kLazy)
 constexpr int kSlots = 3;       // K / V^T blocks resident in LDS (block j in slot j % 3)
 
@@ -60,6 +58,11 @@ struct AttnParams {
     int64_t q_ts, q_hs, k_ts, k_hs, v_ts, v_hs, o_ts, o_hs;
     int tokens;
     float c;   // scale * log2(e)
+    int q_first;   // first query of the launch
+    // key splits: split sp of a batch item sees key blocks sp * split_blocks ... (splits = 1: all of them)
+    int splits, split_blocks;
+    float* part;   // PART: [splits][batch * heads][tokens - q_first] rows of 64 unnormalised outputs
+    float* ml;     // PART: as many (reference maximum, weight sum) pairs
 };
 
 __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
@@ -71,12 +74,14 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
 }
 
-// QS sets of 32 queries per wave, 8 waves (256 * QS queries per workgroup); every K and V^T
-// fragment read from LDS feeds the MFMAs of all QS sets.  Waves 0-3 move each K / V block
-// into LDS for all 8 (half the per-query load and transpose work of 4-wave workgroups).
-template <int QS>
-__global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
-    constexpr int BQ = 256 * QS;
+// QS sets of 32 queries per wave, NW waves (8 or 4; 32 * NW * QS queries per workgroup); every K and V^T
+// fragment read from LDS feeds the MFMAs of all QS sets (two sets: 233 VGPRs, 2 waves per SIMD; one: 150, 3
+// waves).  Waves 0-3 move each K / V block into LDS for all 8 (half the per-query load and transpose work of
+// 4-wave workgroups).  Every query goes through the same operations in the same order whatever QS and NW are.
+// PART: one split of the keys, its unnormalised outputs and (m_ref, sum) pairs to p.part / p.ml (fp32).
+template <int QS, int NW, bool PART>
+__global__ __launch_bounds__(64 * NW) void fmha_d64(AttnParams p) {
+    constexpr int BQ = 32 * NW * QS;
     constexpr int KV = kBK * kD;                                      // elements of one K or V^T block
     __shared__ __attribute__((aligned(16))) uint16_t ks[kSlots * KV];   // [slot][key][dim]
     __shared__ __attribute__((aligned(16))) uint16_t vt[kSlots * KV];   // [slot][dim][key]
@@ -84,10 +89,10 @@ __global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar)
-    const int h = blockIdx.y, b = blockIdx.z;
+    const int h = blockIdx.y, b = PART ? blockIdx.z / p.splits : blockIdx.z;
     const int n = p.tokens;
     const int64_t row0 = (int64_t)b * n;                 // first token row of this batch item
-    const int q0 = blockIdx.x * BQ + wave * 32 * QS;   // the wave's first query
+    const int q0 = p.q_first + blockIdx.x * BQ + wave * 32 * QS;   // the wave's first query
     const int hi = lane >> 5;                           // which 8 of a 16-wide k chunk this lane holds
     const bool wave_active = q0 < n;                    // wave-uniform
 
@@ -182,7 +187,10 @@ __global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
     }
     const float thr = kLazy / p.c;   // raw-score margin of the lazy maximum
 
-    const int nblk = (n + kBK - 1) / kBK;
+    const int sp = PART ? (int)blockIdx.z % p.splits : 0;
+    const int j0 = sp * p.split_blocks;                   // this workgroup's key blocks: j0 .. nblk - 1
+    const int nall = (n + kBK - 1) / kBK;
+    const int nblk = PART && j0 + p.split_blocks < nall ? j0 + p.split_blocks : nall;
     const bool loader = tid < kThreads;                   // waves 0-3 (wave-uniform)
 
     // S = K . Q^T for the 64 keys of block j (two 32-key halves), each K fragment used by every set;
@@ -312,11 +320,11 @@ __global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
     __builtin_amdgcn_s_waitcnt(0);
     uint32_t pk[QS][2][8];                                // [set][half][g * 2 + dword]
     if (loader) {
-        load_block(0);
+        load_block(j0 * kBK);
         store_block(0);
-        if (nblk > 1) load_block(kBK);
+        if (j0 + 1 < nblk) load_block((j0 + 1) * kBK);
         int slot = 0;                                     // slot of block j
-        for (int j = 0; j < nblk; ++j) {
+        for (int j = j0; j < nblk; ++j) {
             __syncthreads();                              // block j stored; blocks before j - 1 no longer read
             const int nslot = slot == kSlots - 1 ? 0 : slot + 1;
             if (j + 1 < nblk) {
@@ -335,10 +343,10 @@ __global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
         }
     } else {
         int slot = 0, pslot = 0;                          // slots of blocks j and j - 1
-        for (int j = 0; j < nblk; ++j) {
+        for (int j = j0; j < nblk; ++j) {
             __syncthreads();
             if (wave_active) {
-                if (j > 0) pv(pslot, pk);
+                if (j > j0) pv(pslot, pk);
                 f32x16 s[QS][2];
                 scores(j, slot, s);
                 softmax(s, pk);
@@ -354,6 +362,22 @@ __global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
     for (int qs = 0; qs < QS; ++qs) {
         const int qi = q0 + 32 * qs + (lane & 31);
         const float l_tot = l_run[qs] + __shfl_xor(l_run[qs], 32, 64);
+        if constexpr (PART) {
+            if (qi < n) {
+                const int64_t row = ((int64_t)(sp * (gridDim.z / p.splits) + b) * gridDim.y + h) * (n - p.q_first) +
+                                    (qi - p.q_first);
+                float* dst = p.part + row * kD + 4 * hi;
+#pragma unroll
+                for (int db = 0; db < 2; ++db)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        *reinterpret_cast<float4*>(dst + 32 * db + 8 * g) =
+                            make_float4(oacc[qs][db][4 * g], oacc[qs][db][4 * g + 1], oacc[qs][db][4 * g + 2],
+                                        oacc[qs][db][4 * g + 3]);
+                if (hi == 0) *reinterpret_cast<float2*>(p.ml + 2 * row) = make_float2(m_ref[qs], l_tot);
+            }
+            continue;
+        }
         const float inv = 1.0f / l_tot;
         if (qi < n) {
             uint16_t* dst = p.o + (row0 + qi) * p.o_ts + h * p.o_hs + 4 * hi;
@@ -370,17 +394,97 @@ __global__ __launch_bounds__(2 * kThreads) void fmha_d64(AttnParams p) {
     }
 }
 
+// Merge of the key splits: per query the splits' outputs and sums rescaled to their largest reference maximum,
+// added in split order, normalised.  16 threads per query, 4 dims each.
+__global__ __launch_bounds__(256) void fmha_merge(AttnParams p, int heads, int64_t rows) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = i >> 4;
+    if (row >= rows) return;
+    const int d = 4 * (int)(i & 15);
+    float m = -__builtin_inff();
+    for (int sp = 0; sp < p.splits; ++sp) m = __builtin_fmaxf(m, p.ml[2 * (sp * rows + row)]);
+    float l = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int sp = 0; sp < p.splits; ++sp) {
+        const float2 ml = *reinterpret_cast<const float2*>(p.ml + 2 * (sp * rows + row));
+        const float4 v = *reinterpret_cast<const float4*>(p.part + (sp * rows + row) * kD + d);
+        const float w = ml.x == m ? 1.0f : __builtin_amdgcn_exp2f((ml.x - m) * p.c);
+        l += w * ml.y;
+        o[0] += w * v.x; o[1] += w * v.y; o[2] += w * v.z; o[3] += w * v.w;
+    }
+    const float inv = 1.0f / l;
+    const int rest = p.tokens - p.q_first;
+    const int64_t bh = row / rest;
+    const int64_t t = (bh / heads) * p.tokens + p.q_first + row % rest;
+    u16x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = f2h(o[e] * inv);
+    *reinterpret_cast<u16x4*>(p.o + t * p.o_ts + (bh % heads) * p.o_hs + d) = y;
+}
+
+// Launches of one attention call: queries [0, head) as the workgroup shape `shape`, then the rest as 256-query
+// workgroups (one set per wave), their keys split `splits` ways.
+enum class AttnShape { Q512, Q256, Q256x4, Q128 };   // 8 waves x 2 sets, 8 x 1, 4 x 2, 4 x 1
+struct AttnPlan {
+    AttnShape shape;
+    int64_t head;       // a multiple of 512, or tokens
+    int splits, split_blocks;
+};
+
+// A CU holds one 8-wave workgroup of two sets, so the count of 512-query workgroups t against the 256 CUs
+// decides (us for 512 / 256 / 256 on 4 waves / 128 queries; batch x tokens x 32 heads):
+//   t <= 64          128 queries            1 x 453: 22.9 / 15.3 / 17.3 / 12.3, 1 x 1013: 38.1 / 26.0 / 29.9 / 22.2
+//   t <= 128         256 queries            1 x 1797: 63.8 / 46.9 / 51.4 / 50.9, 4 x 453: 24.5 / 17.6 / 20.5 / 21.2
+//   t <= 256         512 queries            2 x 1797: 75.0 / 87.9 / 85.2 / 92.7
+// Beyond one round, workgroups of 512 for the whole rounds; the queries past them, when they are at most 128
+// workgroups of 256 queries and the full rounds are nearly full, run with their keys split so that they fill the
+// chip too (1 x 8405: 825.6 -> 651.7; 1 x 4100: 277.3 -> 179.1; error against 64 bits unchanged, 2.96e-4).  Otherwise 4-wave workgroups, two of which share a
+// CU, where the last round is under 3/4 full (3 x 1797: 133.5 / 128.8 / 125.7 / 130.7; 1 x 7173, 15/16 full:
+// 495.2 / 587.7 / 559.3 / 620.6).
+AttnPlan plan_attention(int64_t batch, int64_t tokens, int64_t heads, bool may_split) {
+    constexpr int64_t kCUs = 256;
+    const int64_t bh = batch * heads, nblk = (tokens + kBK - 1) / kBK;
+    const int64_t t = (tokens + 511) / 512 * bh;
+    AttnPlan plan = {AttnShape::Q512, tokens, 1, (int)nblk};
+    if (t <= 64) plan.shape = AttnShape::Q128;
+    else if (t <= 128) plan.shape = AttnShape::Q256;
+    if (t <= kCUs || t % kCUs == 0) return plan;
+    const int64_t rounds = t / kCUs, full = rounds * kCUs / bh;   // 512-query blocks per head in whole rounds
+    const int64_t rest = tokens - 512 * full, w = (rest + 255) / 256 * bh;
+    if (full > 0 && 16 * full * bh >= 15 * rounds * kCUs && w <= 128) {
+        // at least 4 key blocks a split (tokens > 512 here, so a split always has some)
+        int64_t splits = may_split ? kCUs / w : 1;
+        splits = splits < nblk / 4 ? splits : nblk / 4;
+        splits = splits < 1 ? 1 : (splits > 16 ? 16 : splits);
+        plan.head = 512 * full;
+        plan.split_blocks = (int)((nblk + splits - 1) / splits);
+        plan.splits = (int)((nblk + plan.split_blocks - 1) / plan.split_blocks);
+        return plan;
+    }
+    if (4 * (t - rounds * kCUs) < 3 * kCUs) plan.shape = AttnShape::Q256x4;
+    return plan;
+}
+
+int64_t attention_ws_floats(const AttnPlan& plan, int64_t batch, int64_t tokens, int64_t heads) {
+    return plan.splits > 1 ? plan.splits * batch * heads * (tokens - plan.head) * (kD + 2) : 0;
+}
+
+template <int QS, int NW, bool PART>
+void launch_fmha(const AttnParams& p, int64_t queries, int64_t heads, int64_t batch, hipStream_t stream) {
+    constexpr int64_t BQ = 32 * NW * QS;
+    const dim3 grid((unsigned)((queries + BQ - 1) / BQ), (unsigned)heads, (unsigned)(batch * p.splits));
+    hipLaunchKernelGGL((fmha_d64<QS, NW, PART>), grid, dim3(64 * NW), 0, stream, p);
+}
+
 }  // namespace
 }  // namespace h3v
 
 using namespace h3v;
 
-extern "C" int h3v_attention_d64(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, const uint16_t* k,
-                                 int64_t k_token_stride, int64_t k_head_stride, const uint16_t* v,
-                                 int64_t v_token_stride, int64_t v_head_stride, uint16_t* o, int64_t o_token_stride,
-                                 int64_t o_head_stride, int64_t batch, int64_t tokens, int64_t heads, float scale,
-                                 hipStream_t stream) {
-    const char* what = "h3v_attention_d64";
+static int attention_common(const char* what, const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, const uint16_t* k,
+                            int64_t k_token_stride, int64_t k_head_stride, const uint16_t* v, int64_t v_token_stride,
+                            int64_t v_head_stride, uint16_t* o, int64_t o_token_stride, int64_t o_head_stride,
+                            int64_t batch, int64_t tokens, int64_t heads, float scale, bool may_split,
+                            float* workspace, int64_t workspace_floats, hipStream_t stream) {
     H3V_REQUIRE(q && k && v && o, "%s: null pointer argument", what);
     H3V_REQUIRE(batch > 0 && tokens > 0 && heads > 0, "%s: batch, tokens and heads must be positive", what);
     H3V_REQUIRE(batch <= 65535 && heads <= 65535 && tokens <= (1 << 24), "%s: shape out of range", what);
@@ -400,8 +504,59 @@ extern "C" int h3v_attention_d64(const uint16_t* q, int64_t q_token_stride, int6
     p.o_ts = o_token_stride; p.o_hs = o_head_stride;
     p.tokens = (int)tokens;
     p.c = scale * 1.4426950408889634f;
-    constexpr int QS = kQuerySets;
-    dim3 grid((unsigned)((tokens + 256 * QS - 1) / (256 * QS)), (unsigned)heads, (unsigned)batch);
-    hipLaunchKernelGGL(fmha_d64<QS>, grid, dim3(2 * kThreads), 0, stream, p);
+    const AttnPlan plan = plan_attention(batch, tokens, heads, may_split);
+    const int64_t floats = attention_ws_floats(plan, batch, tokens, heads);
+    H3V_REQUIRE(floats == 0 || (workspace && workspace_floats >= floats && aligned(workspace, 16)),
+                "%s: needs a 16-byte aligned workspace of %lld floats", what, (long long)floats);
+    p.q_first = 0;
+    p.splits = 1;
+    p.split_blocks = plan.split_blocks;
+    p.part = p.ml = nullptr;
+    const int64_t head = plan.head;
+    if (plan.shape == AttnShape::Q128) launch_fmha<1, 4, false>(p, head, heads, batch, stream);
+    else if (plan.shape == AttnShape::Q256) launch_fmha<1, 8, false>(p, head, heads, batch, stream);
+    else if (plan.shape == AttnShape::Q256x4) launch_fmha<2, 4, false>(p, head, heads, batch, stream);
+    else launch_fmha<2, 8, false>(p, head, heads, batch, stream);
+    const int64_t rest = tokens - head;
+    if (rest > 0) {
+        p.q_first = (int)head;
+        if (plan.splits == 1) {
+            launch_fmha<1, 8, false>(p, rest, heads, batch, stream);
+        } else {
+            const int64_t rows = batch * heads * rest;
+            p.splits = plan.splits;
+            p.part = workspace;
+            p.ml = workspace + plan.splits * rows * kD;
+            launch_fmha<1, 8, true>(p, rest, heads, batch, stream);
+            hipLaunchKernelGGL(fmha_merge, dim3((unsigned)((rows * 16 + 255) / 256)), dim3(256), 0, stream, p, (int)heads,
+                               rows);
+        }
+    }
     return launch_status(what);
+}
+
+extern "C" int h3v_attention_d64(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, const uint16_t* k,
+                                 int64_t k_token_stride, int64_t k_head_stride, const uint16_t* v,
+                                 int64_t v_token_stride, int64_t v_head_stride, uint16_t* o, int64_t o_token_stride,
+                                 int64_t o_head_stride, int64_t batch, int64_t tokens, int64_t heads, float scale,
+                                 hipStream_t stream) {
+    return attention_common("h3v_attention_d64", q, q_token_stride, q_head_stride, k, k_token_stride, k_head_stride, v,
+                            v_token_stride, v_head_stride, o, o_token_stride, o_head_stride, batch, tokens, heads,
+                            scale, false, nullptr, 0, stream);
+}
+
+extern "C" int64_t h3v_attention_d64_workspace_floats(int64_t batch, int64_t tokens, int64_t heads) {
+    if (batch <= 0 || tokens <= 0 || heads <= 0 || batch > 65535 || heads > 65535 || tokens > (1 << 24)) return 0;
+    return attention_ws_floats(plan_attention(batch, tokens, heads, true), batch, tokens, heads);
+}
+
+extern "C" int h3v_attention_d64_ws(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, const uint16_t* k,
+                                    int64_t k_token_stride, int64_t k_head_stride, const uint16_t* v,
+                                    int64_t v_token_stride, int64_t v_head_stride, uint16_t* o,
+                                    int64_t o_token_stride, int64_t o_head_stride, int64_t batch, int64_t tokens,
+                                    int64_t heads, float scale, float* workspace, int64_t workspace_floats,
+                                    hipStream_t stream) {
+    return attention_common("h3v_attention_d64_ws", q, q_token_stride, q_head_stride, k, k_token_stride, k_head_stride,
+                            v, v_token_stride, v_head_stride, o, o_token_stride, o_head_stride, batch, tokens, heads,
+                            scale, true, workspace, workspace_floats, stream);
 }

@@ -81,9 +81,12 @@ def attention_d64(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: floa
     _hip.require_gfx950(q.device, "attention_d64")
     b, n, h, d = q.shape
     o = torch.empty((b, n, h, d), device=q.device, dtype=q.dtype)
-    _hip.call("h3v_attention_d64", _hip.ptr(q), q.stride(1), q.stride(2), _hip.ptr(k), k.stride(1), k.stride(2),
+    # queries past the last full round of workgroups split their keys over a workspace of fp32 partial outputs
+    floats = int(_hip.lib().h3v_attention_d64_workspace_floats(b, n, h))
+    ws = torch.empty(floats, device=q.device, dtype=torch.float32) if floats else None
+    _hip.call("h3v_attention_d64_ws", _hip.ptr(q), q.stride(1), q.stride(2), _hip.ptr(k), k.stride(1), k.stride(2),
               _hip.ptr(v), v.stride(1), v.stride(2), _hip.ptr(o), o.stride(1), o.stride(2), b, n, h, float(scale),
-              _hip.stream(q.device))
+              _hip.ptr(ws), floats, _hip.stream(q.device))
     return o
 
 

@@ -148,6 +148,23 @@ int h3v_attention_d64(const uint16_t* q, int64_t q_token_stride, int64_t q_head_
                       int64_t v_head_stride, uint16_t* o, int64_t o_token_stride, int64_t o_head_stride,
                       int64_t batch, int64_t tokens, int64_t heads, float scale, hipStream_t stream);
 
+/* The same attention with a caller workspace (the same call site).  When the
+ * 512-query workgroups of a call leave a nearly empty last round on the 256
+ * CUs, its queries run with their keys split over several workgroups that
+ * write unnormalised fp32 outputs, reference maxima and sums to the
+ * workspace, and a second kernel merges them in split order; the other
+ * queries' results are h3v_attention_d64's bit for bit.  workspace_floats
+ * must be at least h3v_attention_d64_workspace_floats() of the same shape
+ * (16-byte aligned); a shape that does not split ignores it (it may be null). */
+int h3v_attention_d64_ws(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, const uint16_t* k,
+                         int64_t k_token_stride, int64_t k_head_stride, const uint16_t* v, int64_t v_token_stride,
+                         int64_t v_head_stride, uint16_t* o, int64_t o_token_stride, int64_t o_head_stride,
+                         int64_t batch, int64_t tokens, int64_t heads, float scale, float* workspace,
+                         int64_t workspace_floats, hipStream_t stream);
+
+/* fp32 workspace floats h3v_attention_d64_ws needs for this shape: 0 when it does not split. */
+int64_t h3v_attention_d64_workspace_floats(int64_t batch, int64_t tokens, int64_t heads);
+
 /* ---- decoder edge: pixel finalisation ------------------------------------
  * Replaces opt/fp16_finalize.py:24-54 (`finalize_pixels`, its Triton kernel).
  * x: decoded pixels [batch, 3, frames, height, width], fp16 (x_is_f16 = 1,

@@ -124,3 +124,62 @@ def test_attention_rejects_bad_layouts(ops):
         att(odd, odd, odd, 0.125)
     with pytest.raises(ValueError, match="scale"):
         att(qd, qd, qd, 0.0)
+
+
+# (batch, tokens, heads) per workgroup shape and split, at the edges of the rule that picks them; `splits`: whether
+# the queries past the full rounds take the key-split kernel and its merge
+@pytest.mark.parametrize("b,n,h,splits", [
+    (1, 65, 64, False), (1, 1025, 21, False),              # 128-query workgroups
+    (1, 64, 65, False), (2, 453, 40, False),               # 256 queries
+    (1, 300, 129, False), (2, 513, 64, False),             # 512 queries, one full round
+    (1, 600, 150, False), (5, 520, 30, False),             # 4-wave workgroups
+    (4, 1025, 32, True), (2, 2049, 32, True), (2, 2300, 32, True), (1, 4097, 32, True), (1, 4101, 31, True),
+    (1, 8250, 16, True),
+])
+def test_attention_workgroup_shapes_and_key_splits(ops, oracle, b, n, h, splits):
+    print(f"attention shapes [{b}, {n}, {h}, 64]", flush=True)
+    floats = int(ops.hip.lib().h3v_attention_d64_workspace_floats(b, n, h))
+    assert (floats > 0) == splits
+    q, k, v, qd, kd, vd = _qkv(b, n, h, seed=b * 100 + n + h)
+    with torch.inference_mode():
+        out = ops.decoder_fused_qk_rope.attention_d64(qd, kd, vd, 0.125)
+        plain = torch.empty_like(out)
+        ops.hip.call("h3v_attention_d64", ops.hip.ptr(qd), qd.stride(1), qd.stride(2), ops.hip.ptr(kd), kd.stride(1),
+                     kd.stride(2), ops.hip.ptr(vd), vd.stride(1), vd.stride(2), ops.hip.ptr(plain), out.stride(1),
+                     out.stride(2), b, n, h, 0.125, ops.hip.stream(DEV))
+    torch.cuda.synchronize()
+    # a few heads against the oracle (every path sees every head alike), the last queries and the edges
+    heads = sorted({0, h // 2, h - 1})
+    rng = np.random.default_rng(n)
+    queries = np.unique(np.concatenate([[0, 31, 32, 63], np.arange(max(0, n - 6), n), rng.integers(0, n, 24)]) % n)
+    for got in (out, plain):
+        _check(ops, oracle, q[:, :, heads], k[:, :, heads], v[:, :, heads].contiguous(), got[:, :, heads], queries)
+    # the two entries differ in the split queries only, by the order of fp32 sums
+    same = (out == plain).all(dim=3).all(dim=2).all(dim=0)
+    assert bool(same.all()) or (splits and bool(same[:512].all()))
+    assert float((out.float() - plain.float()).abs().max()) < 2e-3
+
+
+def test_attention_key_splits_carry_large_scores(ops, oracle):
+    """Splits whose reference maxima differ by far more than 2^8: key norms rise along the sequence, so the last
+    split holds nearly all the weight and the others' outputs are scaled to nothing."""
+    b, n, h = 2, 2100, 32
+    q, k, v, qd, kd, vd = _qkv(b, n, h, seed=17)
+    k = (k.float() * torch.linspace(0.2, 6.0, n).view(1, n, 1, 1)).half()
+    with torch.inference_mode():
+        out = ops.decoder_fused_qk_rope.attention_d64(qd, k.to(DEV), vd, 0.125)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    queries = np.arange(2040, n)
+    _check(ops, oracle, q[:, :, :2], k[:, :, :2], v[:, :, :2].contiguous(), out[:, :, :2], queries)
+
+
+def test_attention_workspace_is_required_for_splits(ops):
+    b, n, h = 4, 1025, 32
+    x = torch.zeros(b, n, h, 64, dtype=torch.float16, device=DEV)
+    need = int(ops.hip.lib().h3v_attention_d64_workspace_floats(b, n, h))
+    ws = torch.empty(need, dtype=torch.float32, device=DEV)
+    args = (ops.hip.ptr(x), x.stride(1), x.stride(2)) * 4 + (b, n, h, 0.125)
+    for bad in ((None, 0), (ops.hip.ptr(ws), need - 1)):
+        with pytest.raises(ValueError, match="workspace"):
+            ops.hip.call("h3v_attention_d64_ws", *args, *bad, ops.hip.stream(DEV))
