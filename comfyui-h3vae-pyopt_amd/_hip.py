@@ -107,24 +107,30 @@ def call(name: str, *args) -> None:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """The tensor's device address as ctypes takes it for a pointer argument."""
+    return None if t is None else t.data_ptr()
 
 
 def stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current HIP stream of ``device`` (torch's raw handle: a Stream object per launch costs 2 us more)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
-@functools.lru_cache(maxsize=8)
-def _device_arch(index: int) -> str:
-    return str(torch.cuda.get_device_properties(index).gcnArchName)
+@functools.lru_cache(maxsize=None)
+def _index_is_gfx950(index: int) -> bool:
+    """Asked only once the GPU is known to be available; the device behind an index does not change."""
+    return str(torch.cuda.get_device_properties(index).gcnArchName).split(":")[0] == "gfx950"
 
 
 def is_gfx950(device) -> bool:
     device = torch.device(device)
-    if device.type != "cuda" or torch.version.hip is None or not torch.cuda.is_available():
+    if device.type != "cuda" or torch.version.hip is None:
         return False
-    index = torch.cuda.current_device() if device.index is None else device.index
-    return _device_arch(index).split(":")[0] == "gfx950"
+    # a GPU in use is available: torch.cuda.is_available() reads the environment on every call
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
+        return False
+    return _index_is_gfx950(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def require_gfx950(device, what: str) -> None:

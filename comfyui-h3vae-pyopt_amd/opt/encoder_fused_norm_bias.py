@@ -46,11 +46,12 @@ def norm_pack_f16(x, weight, bias, eps, pre_bias=None):
     if not x.is_contiguous(memory_format=torch.channels_last_3d):
         x = x.contiguous(memory_format=torch.channels_last_3d)
     y = torch.empty((b, c, d + 2, h + 2, w + 2), device=x.device, dtype=x.dtype, memory_format=torch.channels_last_3d)
-    stats = torch.empty((b * d, 32, 2), device=x.device, dtype=torch.float32)
-    ws = torch.empty(int(_hip.lib().h3v_gn_norm_pack_f16_workspace_floats(b, c, d, h, w)), device=x.device,
+    # one allocation: the statistics, then the workspace
+    ws = torch.empty(b * d * 64 + int(_hip.lib().h3v_gn_norm_pack_f16_workspace_floats(b, c, d, h, w)), device=x.device,
                      dtype=torch.float32)
+    stats = ws.data_ptr()
     _hip.call("h3v_gn_norm_pack_f16", _hip.ptr(x), _hip.ptr(pre_bias), _hip.ptr(weight), _hip.ptr(bias), float(eps),
-              b, c, d, h, w, _hip.ptr(y), _hip.ptr(stats), _hip.ptr(ws), _hip.stream(x.device))
+              b, c, d, h, w, _hip.ptr(y), stats, stats + b * d * 256, _hip.stream(x.device))
     return y
 
 

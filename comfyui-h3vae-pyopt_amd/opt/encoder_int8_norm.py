@@ -55,14 +55,14 @@ def quantized_temporal_norm_pad(x, weight, bias, eps, *, pre_bias=None, return_s
     qy = torch.empty((1, c, d + 2, h + 2, w + 2), device=x.device, dtype=torch.int8,
                      memory_format=torch.channels_last_3d)
     scale = torch.empty((), device=x.device, dtype=torch.float32)
-    stats = torch.empty((d, 32, 2), device=x.device, dtype=torch.float32)
     nws = int(_hip.lib().h3v_gn_norm_pack_workspace_floats(d, h, w))
-    scratch = torch.empty((1,), device=x.device, dtype=torch.int32)
-    tail = (_hip.ptr(qy), _hip.ptr(scale), _hip.ptr(stats))
+    # one allocation: the statistics, the absmax word (16 bytes) and, without partials, the workspace
+    own = torch.empty((d * 64 + 4 + (nws if partials is None else 0),), device=x.device, dtype=torch.float32)
+    stats, scratch = own.data_ptr(), own.data_ptr() + d * 256
+    tail = (_hip.ptr(qy), _hip.ptr(scale), stats)
     if partials is None:
-        workspace = torch.empty((nws,), device=x.device, dtype=torch.float32)
         _hip.call("h3v_gn_norm_pack_i8", _hip.ptr(x), _hip.ptr(pre_bias), _hip.ptr(weight), _hip.ptr(bias),
-                  float(eps), c, d, h, w, *tail, _hip.ptr(workspace), _hip.ptr(scratch), _hip.stream(x.device))
+                  float(eps), c, d, h, w, *tail, scratch + 16, scratch, _hip.stream(x.device))
     else:
         workspace, chunk = partials
         if (workspace.dtype != torch.float32 or workspace.device != x.device or not workspace.is_contiguous()
@@ -75,8 +75,7 @@ def quantized_temporal_norm_pad(x, weight, bias, eps, *, pre_bias=None, return_s
         if chunk not in (TILE_CHUNK, PIXEL_CHUNK):
             raise ValueError(f"partials chunk must be {TILE_CHUNK} or {PIXEL_CHUNK} (got {chunk})")
         _hip.call("h3v_gn_norm_pack_i8_partials", _hip.ptr(x), _hip.ptr(pre_bias), _hip.ptr(weight), _hip.ptr(bias),
-                  float(eps), c, d, h, w, int(chunk), *tail, _hip.ptr(workspace), _hip.ptr(scratch),
-                  _hip.stream(x.device))
+                  float(eps), c, d, h, w, int(chunk), *tail, _hip.ptr(workspace), scratch, _hip.stream(x.device))
     if return_stats:
-        return qy, scale, stats
+        return qy, scale, own[:d * 64].view(d, 32, 2)
     return qy, scale
