@@ -455,7 +455,7 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
         else convert(std::false_type{});
         const int gcol0 = (EP == Epi::SwiGLU) ? tn * (BN / 2) : n0;
         uint16_t* out = static_cast<uint16_t*>(p.out);
-        // Padded output (PADWO = Wo, a tile of whole output rows of one frame): output pixel (t, i, j) of
+        // Padded output (PADWO = Wo, or -1 for the run-time p.Wo; a tile of one frame): output pixel (t, i, j) of
         // batch item b goes to [b, t + pad_front, i + top, j + left] of [B, Do + pad_front, Ho + top +
         // bottom, Wo + left + right, N], and the reflect border of 0 or 1 per side is written with it: row
         // 1 again as row 0 (top), row Ho - 2 as row Ho + top (bottom), likewise columns.  That is the input
@@ -464,14 +464,15 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
         int oh0 = 0, ow0 = 0;
         uint16_t* tile_out = out;   // padded position of the tile's output pixel (0, 0), channel 0
         constexpr int TWP = TILEW ? TILEW : (PADWO > 0 ? PADWO : 1);   // pixels per tile row
-        if constexpr (PADWO > 0) {
-            const int fpix = p.Ho * PADWO;
+        const int pwo = PADWO > 0 ? PADWO : p.Wo;
+        if constexpr (PADWO != 0) {
+            const int fpix = p.Ho * pwo;
             const int fr = m0 / fpix;
-            oh0 = (m0 - fr * fpix) / PADWO;
-            ow0 = (m0 - fr * fpix) - oh0 * PADWO;
+            oh0 = (m0 - fr * fpix) / pwo;
+            ow0 = (m0 - fr * fpix) - oh0 * pwo;
             const int bi = fr / p.Do, od = fr - bi * p.Do;
             pframe = ((int64_t)bi * (p.Do + p.pad_front) + od + p.pad_front) * (p.Ho + p.pad_top + p.pad_bottom);
-            tile_out = out + ((pframe + oh0 + p.pad_top) * (PADWO + p.pad_left + p.pad_right) + p.pad_left + ow0) * p.ldo;
+            tile_out = out + ((pframe + oh0 + p.pad_top) * (pwo + p.pad_left + p.pad_right) + p.pad_left + ow0) * p.ldo;
         }
         // one 8-column chunk of tile row r (output row grow = gidx(r)); every caller has checked vec_out and N
         auto store_chunk = [&](int r, int grow, int gcol, const u16x8& v) {
@@ -479,16 +480,16 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                 *reinterpret_cast<u16x8*>(out + (int64_t)grow * p.ldo + gcol) = v;
             } else {
                 const int ri = r / TWP, owr = r - ri * TWP, ow = ow0 + owr;
-                const int wp = PADWO + p.pad_left + p.pad_right;
+                const int wp = pwo + p.pad_left + p.pad_right;
                 // a tile spans 512 / TWP rows: the offset from tile_out stays below 2^31 elements
                 *reinterpret_cast<u16x8*>(tile_out + (ri * wp + owr) * (int)p.ldo + gcol) = v;
                 const int oh = oh0 + ri;
                 const bool rt = p.pad_top && oh == 1, rb = p.pad_bottom && oh == p.Ho - 2;
-                const bool cl = p.pad_left && ow == 1, cr = p.pad_right && ow == PADWO - 2;
+                const bool cl = p.pad_left && ow == 1, cr = p.pad_right && ow == pwo - 2;
                 if (rt | rb | cl | cr) {   // border pixels: the reflected copies
                     // padded rows / columns that hold this pixel (-1: none)
                     const int r0 = oh + p.pad_top, r1 = rt ? 0 : -1, r2 = rb ? p.Ho + p.pad_top : -1;
-                    const int c0 = ow + p.pad_left, c1 = cl ? 0 : -1, c2 = cr ? PADWO + p.pad_left : -1;
+                    const int c0 = ow + p.pad_left, c1 = cl ? 0 : -1, c2 = cr ? pwo + p.pad_left : -1;
                     auto put = [&](int pr, int pc) {
                         if (pr >= 0 && pc >= 0)
                             *reinterpret_cast<u16x8*>(out + ((pframe + pr) * wp + pc) * p.ldo + gcol) = v;
@@ -532,7 +533,7 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                 u16x8 gb{};
                 if (p.gn_bias) gb = *reinterpret_cast<const u16x8*>(p.gn_bias + gcol);
                 // tile row r is output row m0 + (r / TILEW) * Wo + r % TILEW: 32-bit element offsets from the
-                // tile's first row (at most 8 * 256 rows of 256 channels)
+                // tile's first row (8 rows of a frame of at most 256 channels)
                 uint16_t* const tile_out = out + (int64_t)m0 * p.ldo + gcol;
                 lds_barrier();   // the output tile is complete in LDS
                 // all pieces from LDS first (with the residual added), then the stores
@@ -661,8 +662,8 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                 p.ldo <= 65536) {
                 // Every column of the tile lies inside N: a thread keeps one 8-column chunk for all its rows,
                 // reads all its pieces from LDS first and stores them from the tile's first output row with
-                // 32-bit element offsets (the tile spans at most 512 consecutive rows, or 8 rows of a frame at
-                // most 256 wide); rows past M (the last tile of a GEMM) are skipped.
+                // 32-bit element offsets (the tile spans at most 512 consecutive rows, or 8 rows of a frame);
+                // rows past M (the last tile of a GEMM) are skipped.
                 constexpr int PER = BM * RCH / NT;
                 const int ch = tid % RCH;
                 uint16_t* const tile_out = out + (int64_t)m0 * p.ldo + gcol0 + ch * 8;
@@ -686,7 +687,7 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                     const int grow = gidx(r), gcol = gcol0 + ch * 8;
                     if (grow >= p.M || gcol >= p.N) continue;
                     const u16x8 v = *reinterpret_cast<const u16x8*>(ep + r * (OUTW * 2) + ((ch ^ skey(r)) << 4));
-                    if (PADWO > 0 || (p.vec_out && gcol + 8 <= p.N)) {
+                    if (PADWO != 0 || (p.vec_out && gcol + 8 <= p.N)) {
                         store_chunk(r, grow, gcol, v);
                     } else {
                         uint16_t* dst = out + (int64_t)grow * p.ldo + gcol;
@@ -826,7 +827,7 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                     rv[i] = *reinterpret_cast<const u16x8*>(p.res + (int64_t)grow * p.ldo + gcol);
             }
             lds_barrier();   // the output tile is complete in LDS
-            if (NT % RCH == 0 && (PADWO > 0 || (p.vec_out && gcol0 + OUTW <= p.N))) {
+            if (NT % RCH == 0 && (PADWO != 0 || (p.vec_out && gcol0 + OUTW <= p.N))) {
                 // every piece is a whole 16-byte chunk and a thread keeps one chunk column: all pieces from
                 // LDS with the residual added first, then the stores
                 const int gcol = gcol0 + (tid % RCH) * 8;
@@ -862,7 +863,7 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                 const int grow = gidx(r), gcol = gcol0 + ch * 8;
                 if (idx >= BM * RCH || grow >= p.M || gcol >= p.N) continue;
                 u16x8 v = *reinterpret_cast<const u16x8*>(ep + r * (OUTW * 2) + ((ch ^ skey(r)) << 4));
-                if (PADWO > 0 || (p.vec_out && gcol + 8 <= p.N)) {
+                if (PADWO != 0 || (p.vec_out && gcol + 8 <= p.N)) {
                     if (p.res_bias) {   // fp16(res + (y + b)): both adds in fp32, one rounding
                         const u16x8 rb = *reinterpret_cast<const u16x8*>(p.res_bias + gcol);
 #pragma unroll
@@ -1620,8 +1621,7 @@ __device__ __forceinline__ int sp_slot(int px, int h) {
 // ES = 2: fp16 operands, v_mfma_f32_32x32x16_f16, fp32 accumulators (16 channels per slice).  Both
 // MFMAs read 16 bytes per lane in the same row / k-half layout, so staging and fragments are shared.
 //
-// SP (strided pixels; int8 dequant or int32 output at WO >= 128, fp16 at WO 64; channel bytes a
-// multiple of 128): row r of a wave's accumulator block i is the wave's tile pixel 4r + i, and each
+// SP (strided pixels; int8 dequant or int32 output, or fp16; channel bytes a multiple of 128): row r of a wave's accumulator block i is the wave's tile pixel 4r + i, and each
 // group of four (4r .. 4r + 3) lies in one output row.  Tap (kh, kw) reads window pixels
 // px0 + i + kw (px0 the group's first column): block i of tap kw is "virtual block" V[i + kw] of
 // the six V[v] = pixels px0 + v (v = 0..5) of window row kh.  One kh's three taps read six A
@@ -1631,16 +1631,17 @@ __device__ __forceinline__ int sp_slot(int px, int h) {
 // kh's first four blocks load into base + 6 .. base + 9 while it runs, as many registers as the
 // plain double buffer.
 //
-// TW < WO (with SP: column blocks of 64 pixels): the window of a tile is RO + 2 = 10 rows of 66
-// pixels instead of 4 rows of 258 at Wo 256: 6 window DMA instructions per issuing wave and stage
-// instead of 9.  A wave's 128 pixels are two rows of the block.
+// The SP kernel works on column blocks of TW = 64 pixels of a frame of any width p.Wo that is a multiple of 64
+// (WO = 0: run time): the window of a tile is RO + 2 = 10 rows of 66 pixels instead of 4 rows of 258 at Wo 256,
+// 6 window DMA instructions per issuing wave and stage instead of 9.  A wave's 128 pixels are two rows of the
+// block.
 template <int WO, Epi EP, int ES = 1, bool PAD = false, bool SP = false, int TW = WO>
 __global__ __launch_bounds__(512) void conv3_halo_i8(GemmParams p) {
     static_assert((ES == 2) == (EP == Epi::F16Bias), "fp16 operands use the F16Bias epilogue");
     static_assert(!SP || (((ES == 1 && (EP == Epi::Dequant || EP == Epi::Int32)) || (ES == 2 && EP == Epi::F16Bias)) &&
                           (TW % 128 == 0 || 128 % TW == 0)),
                   "strided pixels: waves of whole tile rows");
-    static_assert(TW == WO || (SP && WO % TW == 0), "column blocks: strided-pixel kernel only");
+    static_assert(SP ? WO == 0 && TW == 64 : TW == WO, "column blocks: strided-pixel kernel only");
     using Acc = std::conditional_t<ES == 1, v16i, f32x16>;
     constexpr int BM = 512, BN = 128, WGM = 4, WGN = 2, NWD = 4;
     constexpr int WM = BM / WGM, WN = BN / WGN;
@@ -1654,7 +1655,7 @@ __global__ __launch_bounds__(512) void conv3_halo_i8(GemmParams p) {
     constexpr int STAGE = HB + WB;
     constexpr int NH = HB / 1024 / NWD, NWT = WB / 1024 / NWD; // DMA instructions per issuing wave and stage
     constexpr int LDS = (2 * STAGE > BM * BN * 2 ? 2 * STAGE : BM * BN * 2) + (SP ? kGnLdsBytes : 0);
-    static_assert(WO == 32 || WO == 64 || WO == 128 || WO == 256, "output width");
+    static_assert(SP || WO == 32 || WO == 64 || WO == 128 || WO == 256, "output width");
     static_assert(LDS <= 163840, "LDS");
     static_assert(LDS == halo_lds_bytes(TW, SP), "host and kernel LDS sizes");
     static_assert(NH + NWT < 64, "outstanding DMA must fit vmcnt");
@@ -1677,11 +1678,12 @@ __global__ __launch_bounds__(512) void conv3_halo_i8(GemmParams p) {
     int id = xcd_remap(blockIdx.x, gridDim.x);
     const int tn = id % p.tiles_n;
     id /= p.tiles_n;
-    const int nfr = p.M / (p.Ho * WO);                        // batch * Do
-    constexpr int NCB = WO / TW;                              // column blocks per output row
+    const int wo = SP ? p.Wo : WO;
+    const int nfr = p.M / (p.Ho * wo);                        // batch * Do
+    const int ncb = SP ? wo / TW : 1;                         // column blocks per output row
     const int rbg = p.tiles_n >= 8 ? 1 : 8 / p.tiles_n;       // row blocks per group
     const int nrb = p.Ho / RO;
-    const int gsz = rbg * nfr * NCB;
+    const int gsz = rbg * nfr * ncb;
     const int rg = id / gsz;
     int rem = id - rg * gsz;
     const int rbn = nrb - rg * rbg < rbg ? nrb - rg * rbg : rbg;
@@ -1693,7 +1695,7 @@ __global__ __launch_bounds__(512) void conv3_halo_i8(GemmParams p) {
     const int bi = fr / p.Do;
     const int oh0 = rb * RO;
     const int owb = cb * TW;                                  // first output column of the tile
-    const int m0 = (fr * p.Ho + oh0) * WO + owb;
+    const int m0 = (fr * p.Ho + oh0) * wo + owb;
     const int n0 = tn * BN;
     const int CB = p.C * ES;                                  // bytes per pixel
     const int CQ = CB / 32;                                   // 32-byte channel slices
@@ -1882,7 +1884,7 @@ __global__ __launch_bounds__(512) void conv3_halo_i8(GemmParams p) {
             run_stage(std::integral_constant<int, 2>{}, s + 2);
             run_stage(std::integral_constant<int, 3>{}, s + 3);
         }
-        write_tile<BM, BN, WGM, WGN, LDS, EP, (PAD ? WO : 0), true, (TW < WO ? TW : 0)>(p, acc, smem, m0, n0, tn);
+        write_tile<BM, BN, WGM, WGN, LDS, EP, (PAD ? -1 : 0), true, TW>(p, acc, smem, m0, n0, tn);
         return;
     }
 
@@ -2090,7 +2092,15 @@ bool halo_conv_fits(const GemmParams& p, int es = 1) {
     return shape && aligned(p.a, 16) && aligned(p.b, 16) && (int64_t)p.Hp * p.Wp * p.C * es * 3 < ((int64_t)1 << 31);
 }
 
-enum class F16Kind { Halo256, Halo128, Halo64, Halo32, Tiled512x128, Tiled256x128, Tiled256x256, Tiled256x128k64,
+// Whether a stride-1 3x3x3 convolution with ES-byte elements takes the strided-pixel kernel: whole 8-row tiles of
+// 64-pixel column blocks and stages in groups of four (C * ES % 128 == 0).
+bool cols_conv_fits(const GemmParams& p, int es = 1) {
+    const bool shape = p.KH == 3 && p.KW == 3 && p.K == 27 * p.C && p.SD == 1 && p.SH == 1 && p.SW == 1 &&
+                       (p.C * es) % 128 == 0 && p.N % 128 == 0 && p.Wo % 64 == 0 && p.Ho % 8 == 0;
+    return shape && aligned(p.a, 16) && aligned(p.b, 16) && (int64_t)p.Hp * p.Wp * p.C * es * 3 < ((int64_t)1 << 31);
+}
+
+enum class F16Kind { Cols, Halo256, Halo128, Halo64, Halo32, Tiled512x128, Tiled256x128, Tiled256x256, Tiled256x128k64,
                      Tiled256x256k64, Tiled256x128k64r3 };
 struct F16Plan {
     F16Kind kind;
@@ -2117,6 +2127,10 @@ F16Plan plan_conv_f16(const GemmParams& p, bool may_split) {
         if (p.Wo == 64) return {F16Kind::Halo64, 1};
         return {F16Kind::Halo32, 1};
     }
+    // Column blocks at any width (17 frames, us, implicit GEMM against it: 128 -> 128 at 480 x 640 4075.4 / 3551.6,
+    // 256 -> 256 at 240 x 320 3664.9 / 3406.8, 9 frames at 128 x 192 632.7 / 594.2); under 128 of these tiles the
+    // implicit GEMM's split reduction fills the chip better.
+    if ((int64_t)p.M / 512 * (p.N / 128) >= 128 && cols_conv_fits(p, 2)) return {F16Kind::Cols, 1};
     const int cb = p.C * 2;
     const int64_t kb = (int64_t)p.K * 2;
     const int64_t m256 = (p.M + 255) / 256;
@@ -2155,14 +2169,14 @@ F16Plan plan_conv_f16(const GemmParams& p, bool may_split) {
     return {F16Kind::Tiled256x256k64, 1};
 }
 
-template <int WO, Epi EP, int ES = 1, bool PAD = false>
-int launch_halo(GemmParams p, hipStream_t stream, const char* what) {
+// Operand extents and epilogue forms of a window convolution.
+template <int ES, bool PAD>
+int fill_halo(GemmParams& p, const char* what) {
     p.tiles_m = p.M / 512;
     p.tiles_n = p.N / 128;
     p.vec_epi = (p.sw == nullptr || aligned(p.sw, 16)) && (p.bias == nullptr || aligned(p.bias, 8)) && p.N % 4 == 0;
     p.vec_out = aligned(p.out, 16) && (p.res == nullptr || aligned(p.res, 16)) && p.ldo % 8 == 0;
     p.conv_tpf = 0;
-    const int64_t grid = (int64_t)p.tiles_m * p.tiles_n;
     const int64_t a_bytes = (int64_t)(p.M / ((int64_t)p.Do * p.Ho * p.Wo)) * p.Dp * p.Hp * p.Wp * p.C * ES;
     const int64_t b_bytes = (int64_t)p.N * p.K * ES;
     if (a_bytes >= ((int64_t)1 << 32) || b_bytes >= ((int64_t)1 << 31))
@@ -2171,26 +2185,41 @@ int launch_halo(GemmParams p, hipStream_t stream, const char* what) {
     p.a_bytes = (uint32_t)a_bytes;
     p.b_bytes = (uint32_t)b_bytes;
     if (PAD && !p.vec_out) return fail(H3V_EINVAL, "%s: the padded output needs 16-byte aligned out and residual", what);
-    // the strided-pixel variant where it applies (int8 dequant or int32 at Wo 128 or 256, fp16 at Wo 64;
-    // stages in groups of four), on column blocks of 64 pixels
-    constexpr bool kSp = (ES == 1 && (EP == Epi::Dequant || EP == Epi::Int32) && WO >= 128) ||
-                         (ES == 2 && EP == Epi::F16Bias && WO == 64);
-    constexpr int kTw = kSp ? 64 : WO;
-    constexpr int lds = halo_lds_bytes(WO, false), lds_sp = halo_lds_bytes(kTw, true);
-    static_assert(lds <= 163840 && lds_sp <= 163840, "LDS exceeds 160 KB");
-    const bool sp = kSp && (p.C * ES) % 128 == 0 && p.Ho % (512 / kTw) == 0;   // whole 8-row tiles of the column blocks
-    if (p.gn_avg && !sp) return fail(H3V_EINVAL, "%s: the statistics epilogue needs the strided-pixel kernel", what);
-    auto kernel = sp ? &conv3_halo_i8<WO, EP, ES, PAD, kSp, kTw> : &conv3_halo_i8<WO, EP, ES, PAD, false>;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv3_halo_i8<WO, EP, ES, PAD, false>),
+    return H3V_OK;
+}
+
+template <Epi EP, int ES = 1, bool PAD = false>
+int launch_cols(GemmParams p, hipStream_t stream, const char* what) {
+    const int rc = fill_halo<ES, PAD>(p, what);
+    if (rc) return rc;
+    constexpr int lds = halo_lds_bytes(64, true);
+    static_assert(lds <= 163840, "LDS exceeds 160 KB");
+    auto kernel = &conv3_halo_i8<0, EP, ES, PAD, true, 64>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    static const hipError_t attr_sp =
-        kSp ? hipFuncSetAttribute(reinterpret_cast<const void*>(&conv3_halo_i8<WO, EP, ES, PAD, kSp, kTw>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_sp)
-            : hipSuccess;
-    const hipError_t ae = attr != hipSuccess ? attr : attr_sp;
-    if (ae != hipSuccess) return fail(H3V_ELAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, sp ? lds_sp : lds,
-                                      hipGetErrorString(ae));
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), sp ? lds_sp : lds, stream, p);
+    if (attr != hipSuccess) return fail(H3V_ELAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds,
+                                        hipGetErrorString(attr));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), lds, stream, p);
+    return launch_status(what);
+}
+
+// Window convolution of a geometry that halo_conv_fits takes: the strided-pixel kernel where it applies (fp16 at
+// 128 -> 128, 17 x 256 x 256 against the plain one: 818.2 -> 767.0 us, 256 -> 256 at 128 x 128: 774.0 -> 746.5), otherwise
+// (64 channel bytes, or output widths 32 and, with int8, 64) the plain one on whole output rows.
+template <int WO, Epi EP, int ES = 1, bool PAD = false>
+int launch_halo(GemmParams p, hipStream_t stream, const char* what) {
+    if (cols_conv_fits(p, ES) && (ES == 2 || WO >= 128)) return launch_cols<EP, ES, PAD>(p, stream, what);
+    if (p.gn_avg) return fail(H3V_EINVAL, "%s: the statistics epilogue needs the strided-pixel kernel", what);
+    const int rc = fill_halo<ES, PAD>(p, what);
+    if (rc) return rc;
+    constexpr int lds = halo_lds_bytes(WO, false);
+    static_assert(lds <= 163840, "LDS exceeds 160 KB");
+    auto kernel = &conv3_halo_i8<WO, EP, ES, PAD, false>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return fail(H3V_ELAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds,
+                                        hipGetErrorString(attr));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(512), lds, stream, p);
     return launch_status(what);
 }
 
@@ -2333,6 +2362,10 @@ int run_conv(GemmParams p, hipStream_t stream, const char* what) {
         if (p.Wo == 64) return launch_halo<64, EP>(p, stream, what);
         return launch_halo<32, EP>(p, stream, what);
     }
+    // Other widths of whole column blocks run on the window kernel too (17 frames, us, implicit GEMM against it:
+    // 128 -> 128 at 480 x 640 2143.5 / 1915.5, at 128 x 192 185.5 / 188.0; 256 -> 256 at 240 x 320 1843.8 / 1712.3,
+    // at 96 x 192 452.6 / 429.4), from 128 tiles on as above.
+    if (halo_tiles >= 128 && cols_conv_fits(p)) return launch_cols<EP>(p, stream, what);
     if (al && p.C % 128 == 0) {
         if (p.N <= 128) return launch_tiled<512, 128, 128, 4, 2, 2, 2, AMode::Conv, EP>(p, stream, what);
         return launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, EP>(p, stream, what);
@@ -2537,6 +2570,7 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
                 "%s: requires Cin %% 32 == 0 and 16-byte aligned x and w (got Cin %d)", what, cin);
     const F16Plan plan = plan_conv_f16(p, may_split);
     switch (plan.kind) {
+        case F16Kind::Cols: return launch_cols<Epi::F16Bias, 2>(p, stream, what);
         case F16Kind::Halo256: return launch_halo<256, Epi::F16Bias, 2>(p, stream, what);
         case F16Kind::Halo128: return launch_halo<128, Epi::F16Bias, 2>(p, stream, what);
         case F16Kind::Halo64: return launch_halo<64, Epi::F16Bias, 2>(p, stream, what);

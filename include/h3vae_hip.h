@@ -94,8 +94,9 @@ int h3v_gn_norm_pack_f16(const uint16_t* x, const uint16_t* pre_bias, const uint
  * item skip the depth taps that read the two leading zero frames.  Requires
  * cin % 32 == 0 and 16-byte aligned x and w.  Stride-1 3x3x3 convs with
  * cout % 128 == 0, an output width of 32, 64, 128 or 256 and an output height
- * that is a multiple of 512 / width run with the input window in LDS; others
- * as an implicit GEMM. */
+ * that is a multiple of 512 / width (or, with cin % 64 == 0 and enough tiles,
+ * any width that is a multiple of 64 and height that is a multiple of 8) run
+ * with the input window in LDS; others as an implicit GEMM. */
 int h3v_conv3d_f16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, const uint16_t* residual,
                    uint16_t* out, int batch, int cin, int d, int h, int wd, int cout, int kd, int kh, int kw, int sd,
                    int sh, int sw, int causal_skip, hipStream_t stream);
