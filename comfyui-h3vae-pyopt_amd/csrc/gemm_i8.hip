@@ -969,36 +969,37 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
         boff[j] = (uint32_t)((int64_t)wrow * p.K + ((lslot ^ swz<BK>(r)) << 4));
     }
 
-    // K blocks of this workgroup: split blockIdx.y of k_splits (the whole K without a split), minus the
-    // causal-zero taps of a conv tile's first frames
+    // K blocks of this workgroup.  The K blocks of one depth tap are `third` (all of them for a GEMM); split
+    // blockIdx.y of k_splits takes the blocks from kin on of every depth tap, `mine` of each, so the splits stay even
+    // when a conv tile of the first frames skips its causal-zero depth taps, and add up the same numbers.
     const int nsplit = p.k_splits > 1 ? p.k_splits : 1;
-    const int kper = p.K / BK / nsplit;
-    const int kend = (int)blockIdx.y * kper + kper;
-    int kb0 = (int)blockIdx.y * kper;
+    int third = p.K / BK, ntap = 1, tap0 = 0;                 // depth taps and the first one that is not skipped
     if constexpr (AM == AMode::Conv) {
-        const int skip = conv_first_kblock(p, m0, BM, BK);
-        kb0 = skip > kb0 ? skip : kb0;
+        third = p.KH * p.KW * p.C / BK;
+        ntap = p.K / BK / third;
+        tap0 = conv_first_kblock(p, m0, BM, BK) / third;
     }
-    const int nk = kend > kb0 ? kend - kb0 : 0;
+    const int per = (third + nsplit - 1) / nsplit;
+    const int kin = (int)blockIdx.y * per;
+    const int mine = third - kin < per ? third - kin : per;   // may be <= 0 in the last splits
+    const int nk = mine > 0 ? (ntap - tap0) * mine : 0;
 
-    // A stages are issued strictly in order, so the conv's k offset is kept as a
-    // running (kd, kh, kw, c0) position advanced by BK per issue: no integer
-    // division in the loop.
-    int ck_kd = 0, ck_kh = 0, ck_kw = 0, ck_c0 = 0;
+    // A and B stages are issued strictly in order, so their k positions are kept running: no integer division
+    // in the loop.  The conv's A position is (kd, kh, kw, c0).
+    int ck_kd = tap0, ck_kh = 0, ck_kw = 0, ck_c0 = 0, a_left = mine;
     if constexpr (AM == AMode::Conv) {
-        const int k0 = kb0 * BK;
-        const int tap = k0 / p.C;
-        ck_c0 = k0 - tap * p.C;
-        ck_kd = tap / (p.KH * p.KW);
-        const int rem = tap - ck_kd * p.KH * p.KW;
-        ck_kh = rem / p.KW;
-        ck_kw = rem - ck_kh * p.KW;
+        const int tap = kin * BK / p.C;
+        ck_c0 = kin * BK - tap * p.C;
+        ck_kh = tap / p.KW;
+        ck_kw = tap - ck_kh * p.KW;
     }
+    const int kh_in = ck_kh, kw_in = ck_kw, c_in = ck_c0;
+    int b_blk = tap0 * third + kin, b_left = mine;
     auto issue_a = [&](int it) {
         int8_t* sa = smem + (it % NSA) * A_BYTES;
         int64_t koff;
         if constexpr (AM == AMode::Gemm) {
-            koff = (int64_t)(kb0 + it) * BK;
+            koff = (int64_t)(kin + it) * BK;
         } else {
             koff = (((int64_t)ck_kd * p.Hp + ck_kh) * p.Wp + ck_kw) * p.C + ck_c0;
             ck_c0 += BK;
@@ -1006,11 +1007,15 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
                 ck_c0 = 0;
                 if (++ck_kw == p.KW) {
                     ck_kw = 0;
-                    if (++ck_kh == p.KH) {
-                        ck_kh = 0;
-                        ++ck_kd;
-                    }
+                    ++ck_kh;
                 }
+            }
+            if (--a_left == 0) {                              // this split's blocks of the next depth tap
+                a_left = mine;
+                ++ck_kd;
+                ck_kh = kh_in;
+                ck_kw = kw_in;
+                ck_c0 = c_in;
             }
         }
         if (!dma_wave) return;
@@ -1018,7 +1023,11 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
         for (int j = 0; j < A_PW; ++j) lds_dma16(ra, aoff[j], (uint32_t)koff, sa + (dw * A_PW + j) * 1024);
     };
     auto issue_b = [&](int it) {
-        const int kb = kb0 + it;
+        const int kb = b_blk++;
+        if (--b_left == 0) {
+            b_left = mine;
+            b_blk += third - mine;
+        }
         int8_t* sb = smem + B_RING + (it % NSB) * B_BYTES;
         if (!dma_wave) return;
 #pragma unroll
@@ -2100,8 +2109,8 @@ bool cols_conv_fits(const GemmParams& p, int es = 1) {
     return shape && aligned(p.a, 16) && aligned(p.b, 16) && (int64_t)p.Hp * p.Wp * p.C * es * 3 < ((int64_t)1 << 31);
 }
 
-enum class F16Kind { Cols, Halo256, Halo128, Halo64, Halo32, Tiled512x128, Tiled256x128, Tiled256x256, Tiled256x128k64,
-                     Tiled256x256k64, Tiled256x128k64r3 };
+enum class F16Kind { Cols, Halo256, Halo128, Halo64, Halo32, Tiled512x128, Tiled256x128, Tiled256x256, Tiled192x256,
+                     Tiled256x128k64, Tiled256x256k64, Tiled256x128k64r3 };
 struct F16Plan {
     F16Kind kind;
     int splits;
@@ -2118,10 +2127,54 @@ int f16_splits(int64_t tiles, int kblocks) {
     return best;
 }
 
+// Tile and K split of the fp16 implicit GEMM for N > 128, by an estimate in us of the candidates: 256 x 256 and
+// 192 x 256 tiles, unsplit or with a reduction split of at most one round of the CUs that divides the K blocks and
+// leaves each split at least 8 of them, and unsplit 256 x 128 tiles.  A 256 x 256 tile takes about 1.45 us per
+// block of 128 bytes of K and 8 us around them on a full chip; a 192-row one 3/4 of that and 4% (three instead of
+// four 32-row blocks share a weight fragment), a 256 x 128 one half and 15%; a split's partial sums are written and
+// read at about 5 TB/s, and the second kernel takes 6 us.  Up to three rounds count whole; over more, the tiles'
+// ends drift apart.  `active` is the share of K a tile runs (a causal conv of one frame skips two thirds).
+// Start against now (us, causal): 4 x 512 -> 512 at 5 x 32 x 32 (160 window tiles against 214 of 192 rows) 238.9 ->
+// 225.8, one clip (40 window tiles, six splits) 213.4 -> 78.6, 512 -> 512 at 5 x 60 x 80 (188 tiles of 256 rows,
+// 250 of 192) 284.8 -> 244.2, 512 -> 512 at 1 x 32 x 32 73.8 -> 25.0.
+struct WidePlan {
+    F16Plan plan;
+    double us;
+};
+WidePlan plan_wide_f16(int64_t m, int64_t n, int kblocks, double active, bool may_split) {
+    const double tile = 1.45 * active * kblocks + 8.0;
+    auto rounds = [](int64_t tiles) { return tiles <= 768 ? (double)((tiles + 255) / 256) : tiles / 256.0 + 0.5; };
+    const int64_t tn = (n + 255) / 256, t256 = (m + 255) / 256 * tn, t192 = (m + 191) / 192 * tn;
+    const int64_t t128 = (m + 255) / 256 * ((n + 127) / 128);
+    WidePlan best = {{F16Kind::Tiled256x256, 1}, rounds(t256) * tile};
+    auto offer = [&](F16Kind kind, int splits, double us) {
+        if (us < 0.95 * best.us) best = {{kind, splits}, us};
+    };
+    offer(F16Kind::Tiled256x128, 1, rounds(t128) * 0.575 * tile);
+    offer(F16Kind::Tiled192x256, 1, rounds(t192) * 0.78 * tile);
+    for (int sp = 2; may_split && n % 4 == 0 && sp <= 16; ++sp) {
+        if (kblocks % sp != 0 || kblocks / sp < 8) continue;
+        const double reduce = 6.0 + (double)sp * m * n * 8 / 5e6;
+        if (t256 * sp <= 256) offer(F16Kind::Tiled256x256, sp, tile / sp + reduce);
+        if (t192 * sp <= 256) offer(F16Kind::Tiled192x256, sp, 0.78 * tile / sp + reduce);
+    }
+    return best;
+}
+
 // Kernel, tile and K split of h3v_conv3d_f16 for the geometry in p (C and K in elements; the implicit
 // GEMM counts them in bytes).  Splits only when the caller supplies a workspace (may_split).
 F16Plan plan_conv_f16(const GemmParams& p, bool may_split) {
-    if (halo_conv_fits(p, 2)) {
+    // Under one round of window tiles the implicit GEMM may fill the chip better, with 192-row tiles or a split
+    // reduction (window tiles take 0.92 of a 256 x 256 tile)
+    const int64_t window = (int64_t)p.M / 512 * (p.N / 128);
+    const int blocks = (int)((int64_t)p.K * 2 / 128);
+    // one output frame of a stride-1 kernel three deep: the framework's single images, whose causal convs run one
+    // of the three depth taps (an estimate only, so that it need not know the call's causal_skip)
+    const double active = p.Do == 1 && p.SD == 1 && p.Dp == 3 ? 1.0 / 3.0 : 1.0;
+    bool wide = false;
+    if (may_split && window < 256 && p.C % 64 == 0 && p.N > 128)
+        wide = plan_wide_f16(p.M, p.N, blocks, active, true).us < 0.9 * (1.45 * active * blocks + 8.0) * 0.92;
+    if (!wide && halo_conv_fits(p, 2)) {
         if (p.Wo == 256) return {F16Kind::Halo256, 1};
         if (p.Wo == 128) return {F16Kind::Halo128, 1};
         if (p.Wo == 64) return {F16Kind::Halo64, 1};
@@ -2130,7 +2183,7 @@ F16Plan plan_conv_f16(const GemmParams& p, bool may_split) {
     // Column blocks at any width (17 frames, us, implicit GEMM against it: 128 -> 128 at 480 x 640 4075.4 / 3551.6,
     // 256 -> 256 at 240 x 320 3664.9 / 3406.8, 9 frames at 128 x 192 632.7 / 594.2); under 128 of these tiles the
     // implicit GEMM's split reduction fills the chip better.
-    if ((int64_t)p.M / 512 * (p.N / 128) >= 128 && cols_conv_fits(p, 2)) return {F16Kind::Cols, 1};
+    if (!wide && window >= 128 && cols_conv_fits(p, 2)) return {F16Kind::Cols, 1};
     const int cb = p.C * 2;
     const int64_t kb = (int64_t)p.K * 2;
     const int64_t m256 = (p.M + 255) / 256;
@@ -2148,16 +2201,7 @@ F16Plan plan_conv_f16(const GemmParams& p, bool may_split) {
             if (round_fill((p.M + 511) / 512) < 0.9 * round_fill(m256)) return {F16Kind::Tiled256x128, 1};
             return {F16Kind::Tiled512x128, 1};
         }
-        const int64_t t256 = m256 * ((p.N + 255) / 256);
-        if (may_split && p.N % 4 == 0) {
-            const int sp = f16_splits(t256, kblocks);
-            if (sp > 1) return {F16Kind::Tiled256x256, sp};
-        }
-        // Cout > 128 with so few 256 x 256 tiles that even twice as many fit one round on the 256 CUs
-        // (the 16^2 suffix stage: 80 tiles): 256 x 128 tiles of eight 64 x 64 wave blocks.  At 144 tiles
-        // (the stride-2 downsample) the 288 smaller tiles need a second round and ran 35% slower.
-        if (2 * t256 <= 256) return {F16Kind::Tiled256x128, 1};
-        return {F16Kind::Tiled256x256, 1};
+        return plan_wide_f16(p.M, p.N, kblocks, active, may_split).plan;
     }
     const bool few = p.N > 128 && 2 * m256 * ((p.N + 255) / 256) <= 256;
     // Cout <= 128 with K steps of 64 bytes (conv_in: 32 tap-folded channels x 3 taps): 256 x 128 tiles over
@@ -2592,9 +2636,12 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
         q.bias = nullptr;
         q.res = nullptr;
         q.k_splits = plan.splits;
-        rc = plan.kind == F16Kind::Tiled256x256
-                 ? launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F32Part>(q, stream, what)
-                 : launch_tiled<256, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
+        if (plan.kind == F16Kind::Tiled256x256)
+            rc = launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
+        else if (plan.kind == F16Kind::Tiled192x256)
+            rc = launch_tiled<192, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
+        else
+            rc = launch_tiled<256, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
         if (rc) return rc;
         const int64_t mn = (int64_t)p.M * p.N;
         hipLaunchKernelGGL(splitk_reduce_f16, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream,
@@ -2605,6 +2652,7 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
         case F16Kind::Tiled512x128: return launch_tiled<512, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x128: return launch_tiled<256, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x256: return launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
+        case F16Kind::Tiled192x256: return launch_tiled<192, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x128k64: return launch_tiled<256, 128, 64, 4, 2, 4, 4, AMode::Conv, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x128k64r3: return launch_tiled<256, 128, 64, 4, 2, 3, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
         default: return launch_tiled<256, 256, 64, 2, 4, 4, 4, AMode::Conv, Epi::F16Bias>(p, stream, what);

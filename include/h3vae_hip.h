@@ -102,9 +102,9 @@ int h3v_conv3d_f16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, c
                    int sh, int sw, int causal_skip, hipStream_t stream);
 
 /* The same convolution with a caller workspace for a split reduction (the
- * same model call sites as h3v_conv3d_f16).  When the implicit GEMM would
- * leave most CUs idle (fewer tiles than half a round of the 256 CUs) and K is
- * long, the reduction is split S ways: S workgroups per tile write fp32
+ * same model call sites as h3v_conv3d_f16).  When the conv would leave CUs
+ * idle (under half a round of implicit-GEMM tiles on the 256 CUs, or under a
+ * round of window tiles) and K is long, the reduction is split S ways: S workgroups per tile write fp32
  * partial sums to workspace [S, M, cout], and a second kernel adds them in
  * split order and applies the same epilogue (fp16(sum + bias), then the
  * residual).  The sums' order differs from h3v_conv3d_f16's, the values stay

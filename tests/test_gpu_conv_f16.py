@@ -152,6 +152,10 @@ SPLIT_CASES = [
     (1, 1024, 7, 18, 18, 48, False, False),     # conv_out-like: Cout 48 on 256 x 128 tiles, 16 splits
     (1, 256, 7, 18, 18, 256, False, True),      # 256 x 256 tiles, 12 splits, with a residual
     (2, 256, 5, 18, 18, 256, True, False),      # causal skip: frames 0 / 1 leave whole splits empty
+    (1, 256, 3, 66, 66, 256, True, True),       # one output frame: two of the three depth taps skipped
+    (1, 512, 7, 34, 34, 512, True, False),      # a window-kernel width, split instead
+    (1, 512, 5, 42, 30, 512, True, True),       # 192-row tiles, a last tile across the end
+    (1, 128, 7, 50, 34, 256, False, False),     # window width, K of 54 blocks
 ]
 
 
