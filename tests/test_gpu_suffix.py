@@ -39,7 +39,13 @@ def _oracle(oracle, x, gamma, beta, pb, b, eps):
 
 @pytest.mark.parametrize("c,b,d,h,w,pb", [(128, 1, 3, 6, 9, False), (256, 3, 2, 5, 7, True), (512, 1, 3, 8, 8, False),
                                           (512, 4, 2, 7, 5, True), (1024, 3, 2, 6, 6, False), (1024, 1, 5, 9, 4, True),
-                                          (256, 4, 9, 64, 64, False), (512, 4, 5, 32, 32, True)])
+                                          (256, 4, 9, 64, 64, False), (512, 4, 5, 32, 32, True),
+                                          # rows of one to five times the vectors a block takes, short by one pixel,
+                                          # exact and over; and rows enough for one block each
+                                          (1024, 1, 2, 3, 29, True), (1024, 1, 2, 2, 30, False),
+                                          (1024, 1, 1, 5, 31, True), (512, 1, 2, 3, 62, False),
+                                          (256, 1, 3, 4, 127, True), (128, 1, 1, 4, 190, False),
+                                          (256, 2, 7, 300, 6, True)])
 def test_norm_pack_f16_matches_oracle(ops, oracle, c, b, d, h, w, pb):
     print(f"norm_pack_f16 C={c} B={b} D={d} {h}x{w} pre_bias={pb}", flush=True)
     x, gamma, beta, pre = _inputs(b, c, d, h, w, pb, seed=c + b + d + h + w)
