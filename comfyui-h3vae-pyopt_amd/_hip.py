@@ -37,6 +37,7 @@ SIGNATURES: dict[str, list] = {
     "h3v_gemm_i8_i32": [_P, _P, _P, _I64, _I64, _I64, _P],
     "h3v_conv3d_i8_residual": [_P] * 7 + [_I] * 13 + [_P],
     "h3v_conv3d_i8_residual_padded": [_P] * 8 + [_I] * 12 + [_P],
+    "h3v_conv3d_i8_cols": [_P] * 8 + [_I] * 12 + [_P, _P, _P],
     "h3v_conv3d_i8_gn": [_P] * 7 + [_I] * 6 + [_P, _P, _P],
     "h3v_conv3d_i8": [_P, _P, _P, _P, _P, _P] + [_I] * 13 + [_P],
     "h3v_conv3d_i8_i32": [_P, _P, _P] + [_I] * 13 + [_P],

@@ -969,10 +969,12 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
         boff[j] = (uint32_t)((int64_t)wrow * p.K + ((lslot ^ swz<BK>(r)) << 4));
     }
 
-    // K blocks of this workgroup.  The K blocks of one depth tap are `third` (all of them for a GEMM); split
-    // blockIdx.y of k_splits takes the blocks from kin on of every depth tap, `mine` of each, so the splits stay even
-    // when a conv tile of the first frames skips its causal-zero depth taps, and add up the same numbers.
-    const int nsplit = p.k_splits > 1 ? p.k_splits : 1;
+    // K blocks of this workgroup: all of them past the causal-zero depth taps of a conv tile's first frames.  With a
+    // K split (F32Part): the K blocks of one depth tap are `third`, and split blockIdx.y of k_splits takes the blocks
+    // from kin on of every depth tap, `mine` of each, so the splits stay even when depth taps are skipped, and add up
+    // the same numbers.
+    constexpr bool SPLIT = EP == Epi::F32Part;
+    const int nsplit = SPLIT && p.k_splits > 1 ? p.k_splits : 1;
     int third = p.K / BK, ntap = 1, tap0 = 0;                 // depth taps and the first one that is not skipped
     if constexpr (AM == AMode::Conv) {
         third = p.KH * p.KW * p.C / BK;
@@ -1007,10 +1009,13 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
                 ck_c0 = 0;
                 if (++ck_kw == p.KW) {
                     ck_kw = 0;
-                    ++ck_kh;
+                    if (++ck_kh == p.KH && !SPLIT) {
+                        ck_kh = 0;
+                        ++ck_kd;
+                    }
                 }
             }
-            if (--a_left == 0) {                              // this split's blocks of the next depth tap
+            if (SPLIT && --a_left == 0) {                     // this split's blocks of the next depth tap
                 a_left = mine;
                 ++ck_kd;
                 ck_kh = kh_in;
@@ -1023,8 +1028,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
         for (int j = 0; j < A_PW; ++j) lds_dma16(ra, aoff[j], (uint32_t)koff, sa + (dw * A_PW + j) * 1024);
     };
     auto issue_b = [&](int it) {
-        const int kb = b_blk++;
-        if (--b_left == 0) {
+        const int kb = SPLIT ? b_blk++ : b_blk + it;
+        if (SPLIT && --b_left == 0) {
             b_left = mine;
             b_blk += third - mine;
         }
@@ -2557,6 +2562,48 @@ int h3v_conv3d_i8_gn(const int8_t* qx, const float* x_scale, const int8_t* qw, c
     p.gn_bias = gn_bias;
     p.gn_nchunk = g.nchunk;
     return p.Wo == 256 ? launch_halo<256, Epi::Dequant>(p, stream, what) : launch_halo<128, Epi::Dequant>(p, stream, what);
+}
+
+int h3v_conv3d_i8_cols(const int8_t* qx, const float* x_scale, const int8_t* qw, const float* w_scale,
+                       const uint16_t* bias, const uint16_t* residual, const uint16_t* residual_bias, uint16_t* out,
+                       int cin, int d, int h, int w, int cout, int causal_skip, int padded, int front, int top,
+                       int bottom, int left, int right, const uint16_t* gn_bias, float* workspace,
+                       hipStream_t stream) {
+    const char* what = "h3v_conv3d_i8_cols";
+    H3V_REQUIRE(qx && x_scale && qw && w_scale && out, "%s: null pointer argument", what);
+    H3V_REQUIRE(residual || !residual_bias, "%s: residual_bias needs a residual", what);
+    H3V_REQUIRE(residual != out, "%s: the residual must not alias the output", what);
+    H3V_REQUIRE((padded != 0) != (workspace != nullptr), "%s: writes either the padded output or the statistics", what);
+    H3V_REQUIRE(padded || !residual_bias, "%s: residual_bias is only taken with the padded output", what);
+    H3V_REQUIRE(!padded || (front >= 0 && front <= 16), "%s: front must be in [0, 16] (got %d)", what, front);
+    H3V_REQUIRE(!padded || ((top | bottom | left | right) >= 0 && (top | bottom | left | right) <= 1),
+                "%s: the reflect border is 0 or 1 on each side (got %d, %d, %d, %d)", what, top, bottom, left, right);
+    GemmParams p{};
+    int rc = fill_conv(p, what, 1, cin, d, h, w, cout, 3, 3, 3, 1, 1, 1);
+    if (rc) return rc;
+    p.a = qx; p.b = qw; p.sx = x_scale; p.sx_stride = 0; p.sw = w_scale; p.bias = bias; p.out = out;
+    p.res = residual;
+    p.res_bias = residual_bias;
+    p.causal_skip = causal_skip ? 1 : 0;
+    H3V_REQUIRE(cols_conv_fits(p) && cout <= 65536 && (padded || cout == 128 || cout == 256),
+                "%s: needs Cin %% 128 == 0, Cout %% 128 == 0 (128 or 256 with statistics), an output width that is a "
+                "multiple of 64 and an output height that is a multiple of 8 (got Cin %d, Cout %d, output %d x %d)", what,
+                cin, cout, p.Ho, p.Wo);
+    H3V_REQUIRE(aligned(out, 16) && (!residual || aligned(residual, 16)) && (!residual_bias || aligned(residual_bias, 16)) &&
+                    (!gn_bias || aligned(gn_bias, 16)) && aligned(workspace, 16),
+                "%s: out, residual, residual_bias, gn_bias and workspace need 16-byte alignment", what);
+    if (padded) {
+        p.pad_front = front;
+        p.pad_top = top; p.pad_bottom = bottom; p.pad_left = left; p.pad_right = right;
+        return launch_cols<Epi::Dequant, 1, true>(p, stream, what);
+    }
+    const GnWorkspace g = gn_workspace(workspace, p.Do, p.Ho * p.Wo, kGnTileChunk);
+    p.gn_avg = g.avg;
+    p.gn_m2 = g.m2;
+    p.gn_ext = g.ext;
+    p.gn_bias = gn_bias;
+    p.gn_nchunk = g.nchunk;
+    return launch_cols<Epi::Dequant>(p, stream, what);
 }
 
 int h3v_conv3d_i8_residual_padded(const int8_t* qx, const float* x_scale, const int8_t* qw, const float* w_scale,

@@ -164,8 +164,8 @@ class BiasFusedResidualBlock(torch.nn.Module):
         if consumer is None or self.int8_second is None or not self.int8_second.fuse_norm:
             return None
         from .encoder_int8 import padded_output_fits
-        _, c, _, h, w = out_like.shape
-        if not padded_output_fits(self.int8_second.config.in_channels, c, h, w):
+        b, c, d, h, w = out_like.shape
+        if not padded_output_fits(self.int8_second.config.in_channels, c, h, w, batch=b, out_d=d):
             return None
         return consumer.padded_input_form(out_like)
 

@@ -77,8 +77,9 @@ class ResidualDownsampleBlock(BiasFusedResidualBlock):
         first norm in INT8 mode).  The first conv hands its tile statistics to the second norm."""
         if self.int8_first is not None and self.int8_first.fuse_norm and self.int8_second.fuse_norm:
             from .encoder_int8 import padded_output_fits
-            h, w = x.shape[3:]
-            if padded_output_fits(self.int8_second.config.in_channels, self.int8_second.config.out_channels, h, w):
+            b, _, d, h, w = x.shape
+            if padded_output_fits(self.int8_second.config.in_channels, self.int8_second.config.out_channels, h, w,
+                                  batch=b, out_d=d):
                 # The second conv writes the pack's output itself: fp16(x + (conv + second.bias)) into the
                 # downsample's padded input (two zero frames, bottom / right reflect); bit-identical to the
                 # conv followed by residual_downsample_pack, without re-reading the conv output.

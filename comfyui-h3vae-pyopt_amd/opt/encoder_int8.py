@@ -218,9 +218,14 @@ def _conv3d_from_quantized(qx, activation_scale, qweight, weight_scale, *, confi
         if gn_bias is not None and (gn_bias.shape != (config.out_channels,) or gn_bias.dtype != torch.float16
                                     or gn_bias.device != out.device):
             raise ValueError("gn_bias must be an fp16 vector of the output channels on the output's device")
-        _hip.call("h3v_conv3d_i8_gn", *head, _hip.ptr(residual), _hip.ptr(out), c, d, h, w, config.out_channels,
-                  int(bool(causal_prefix_zero)), _hip.ptr(None if gn_bias is None else gn_bias.contiguous()),
-                  _hip.ptr(gn_workspace), _hip.stream(qx.device))
+        gn_bias = None if gn_bias is None else gn_bias.contiguous()
+        geometry = (c, d, h, w, config.out_channels, int(bool(causal_prefix_zero)))
+        if out_shape[4] in (128, 256):
+            _hip.call("h3v_conv3d_i8_gn", *head, _hip.ptr(residual), _hip.ptr(out), *geometry, _hip.ptr(gn_bias),
+                      _hip.ptr(gn_workspace), _hip.stream(qx.device))
+        else:
+            _hip.call("h3v_conv3d_i8_cols", *head, _hip.ptr(residual), None, _hip.ptr(out), *geometry, 0, 0, 0, 0, 0, 0,
+                      _hip.ptr(gn_bias), _hip.ptr(gn_workspace), _hip.stream(qx.device))
         return out
     if gn_bias is not None:
         raise ValueError("gn_bias is only taken with gn_workspace")
@@ -232,13 +237,13 @@ def _conv3d_from_quantized(qx, activation_scale, qweight, weight_scale, *, confi
 
 
 def gn_stats_fits(in_channels: int, out_channels: int, out_d: int, out_h: int, out_w: int, *, batch: int = 1) -> bool:
-    """Whether ``h3v_conv3d_i8_gn`` takes a stride-1 3x3x3 conv of this geometry and whether it is the
-    kernel the plain conv would run anyway: the window conv's strided-pixel form (batch one, Cin % 128 == 0,
-    Cout 128 or 256, output width 128 or 256, output height a multiple of 8), at 128 or more 512 x 128
-    output tiles (fewer run as the implicit GEMM, which fills the GPU better)."""
+    """Whether ``h3v_conv3d_i8_gn`` or ``h3v_conv3d_i8_cols`` takes a stride-1 3x3x3 conv of this geometry and
+    whether it is the kernel the plain conv would run anyway: the window conv's strided-pixel form (batch one,
+    Cin % 128 == 0, Cout 128 or 256, output width a multiple of 64 from 128, output height a multiple of 8), at
+    128 or more 512 x 128 output tiles (fewer run as the implicit GEMM, which fills the GPU better)."""
     tiles = out_d * (out_h * out_w // 512) * (out_channels // 128)
-    return (batch == 1 and in_channels % 128 == 0 and out_channels in (128, 256) and out_w in (128, 256)
-            and out_d >= 1 and out_h >= 8 and out_h % 8 == 0 and tiles >= 128)
+    return (batch == 1 and in_channels % 128 == 0 and out_channels in (128, 256) and out_w % 64 == 0
+            and out_w >= 128 and out_d >= 1 and out_h >= 8 and out_h % 8 == 0 and tiles >= 128)
 
 
 def gn_workspace_floats(d: int, h: int, w: int) -> int:
@@ -249,12 +254,17 @@ def gn_workspace_floats(d: int, h: int, w: int) -> int:
     return n
 
 
-def padded_output_fits(in_channels: int, out_channels: int, out_h: int, out_w: int) -> bool:
+def padded_output_fits(in_channels: int, out_channels: int, out_h: int, out_w: int, *, batch: int = 1,
+                       out_d: int = 0) -> bool:
     """Whether ``h3v_conv3d_i8_residual_padded`` takes a stride-1 3x3x3 conv of this geometry (the
     window-in-LDS kernel: Cin % 64 == 0, Cout % 128 == 0, output width 32/64/128/256, output height a
-    multiple of 512 / width and at least 2)."""
-    return (in_channels % 64 == 0 and out_channels % 128 == 0 and out_w in (32, 64, 128, 256)
-            and out_h >= 2 and out_h % (512 // out_w) == 0)
+    multiple of 512 / width and at least 2), or, given its ``out_d`` output frames, whether
+    ``h3v_conv3d_i8_cols`` does and is the kernel the plain conv would run (batch one, other widths that are
+    multiples of 64, output height a multiple of 8, at least 128 tiles)."""
+    if in_channels % 64 == 0 and out_channels % 128 == 0 and out_w in (32, 64, 128, 256):
+        return out_h >= 2 and out_h % (512 // out_w) == 0
+    return (batch == 1 and in_channels % 128 == 0 and out_channels % 128 == 0 and out_w >= 128 and out_w % 64 == 0
+            and out_h >= 8 and out_h % 8 == 0 and out_d * (out_h * out_w // 512) * (out_channels // 128) >= 128)
 
 
 def _conv3d_from_quantized_padded(qx, activation_scale, qweight, weight_scale, *, bias, residual, residual_bias,
@@ -282,10 +292,14 @@ def _conv3d_from_quantized_padded(qx, activation_scale, qweight, weight_scale, *
     if residual_bias is not None and (residual is None or tuple(residual_bias.shape) != (cout,)
                                       or residual_bias.dtype != torch.float16):
         raise ValueError("residual_bias needs a residual and must be an fp16 vector of the output channels")
-    _hip.call("h3v_conv3d_i8_residual_padded", _hip.ptr(qx), _hip.ptr(activation_scale), _hip.ptr(qweight),
-              _hip.ptr(weight_scale), _hip.ptr(bias), _hip.ptr(residual),
-              _hip.ptr(None if residual_bias is None else residual_bias.contiguous()), _hip.ptr(out),
-              *qx.shape, cout, 1, int(front), top, bottom, left, right, _hip.stream(qx.device))
+    residual_bias = None if residual_bias is None else residual_bias.contiguous()
+    head = (_hip.ptr(qx), _hip.ptr(activation_scale), _hip.ptr(qweight), _hip.ptr(weight_scale), _hip.ptr(bias),
+            _hip.ptr(residual), _hip.ptr(residual_bias), _hip.ptr(out))
+    border = (int(front), top, bottom, left, right)
+    if b == 1 and wo > 128 and wo != 256 and wo % 64 == 0:
+        _hip.call("h3v_conv3d_i8_cols", *head, *qx.shape[1:], cout, 1, 1, *border, None, None, _hip.stream(qx.device))
+    else:
+        _hip.call("h3v_conv3d_i8_residual_padded", *head, *qx.shape, cout, 1, *border, _hip.stream(qx.device))
     return out
 
 

@@ -283,6 +283,18 @@ int h3v_conv3d_i8_gn(const int8_t* qx, const float* x_scale, const int8_t* qw, c
                      const uint16_t* bias, const uint16_t* residual, uint16_t* out, int cin, int d, int h, int w,
                      int cout, int causal_skip, const uint16_t* gn_bias, float* workspace, hipStream_t stream);
 
+/* The two entries above at any output size of whole 8-row x 64-column tiles
+ * (frames encoded untiled): batch one, wo a multiple of 64, ho a multiple of
+ * 8, cin % 128 == 0, cout % 128 == 0.  Either padded != 0: the padded output
+ * of h3v_conv3d_i8_residual_padded (residual, residual_bias, front and the
+ * border as there; workspace null), or the statistics of h3v_conv3d_i8_gn
+ * (cout 128 or 256; residual, gn_bias and workspace as there; residual_bias
+ * null).  The same model call sites. */
+int h3v_conv3d_i8_cols(const int8_t* qx, const float* x_scale, const int8_t* qw, const float* w_scale,
+                       const uint16_t* bias, const uint16_t* residual, const uint16_t* residual_bias, uint16_t* out,
+                       int cin, int d, int h, int w, int cout, int causal_skip, int padded, int front, int top,
+                       int bottom, int left, int right, const uint16_t* gn_bias, float* workspace, hipStream_t stream);
+
 /* Raw int32 accumulators of the same convolution (exactness checks). */
 int h3v_conv3d_i8_i32(const int8_t* qx, const int8_t* qw, int32_t* acc, int batch, int cin, int d, int h,
                       int w, int cout, int kd, int kh, int kw, int sd, int sh, int sw, int causal_skip,

@@ -2,6 +2,7 @@
 accumulators exactly, and fp16 results within the rounding of their sums, against a float64 convolution."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -51,6 +52,89 @@ def test_int8_exact(ops, b, cin, cout, d, h, w):
     # one fp16 rounding of y (2^-11 |y|), fp32 roundings far below it, one of the sum
     bound = 2.0 ** -11 * (1.01 * y.abs() + (y + res.double()).abs()) + 1e-6
     assert bool(((out.double() - (y + res.double())).abs() <= bound).all())
+
+
+def _operands(cin, cout, d, h, w, seed):
+    gen = torch.Generator(DEV).manual_seed(seed)
+    x = torch.randint(-127, 128, (1, d + 2, h + 2, w + 2, cin), generator=gen, dtype=torch.int8, device=DEV)
+    x[:, :2] = 0
+    wt = torch.randint(-127, 128, (cout, 27 * cin), generator=gen, dtype=torch.int8, device=DEV)
+    sx, sw = torch.tensor(0.004, device=DEV), torch.rand(cout, generator=gen, device=DEV) * 2e-3 + 1e-4
+    bias = (0.2 * torch.randn(cout, generator=gen, device=DEV)).half()
+    res = torch.randn(1, d, h, w, cout, generator=gen, device=DEV).half()
+    return x, wt, sx, sw, bias, res, (0.5 * torch.randn(cout, generator=gen, device=DEV)).half()
+
+
+@pytest.mark.parametrize("cin,cout,d,h,w,with_res,with_bias", [(128, 128, 2, 16, 192, True, False),
+                                                               (128, 256, 3, 8, 64, False, True),
+                                                               (256, 256, 1, 24, 320, True, True),
+                                                               (256, 128, 2, 8, 640, False, False)])
+def test_statistics_at_other_widths(ops, oracle, cin, cout, d, h, w, with_res, with_bias):
+    """h3v_conv3d_i8_cols: the output of the plain conv, and the tile statistics of the oracle, bit for bit."""
+    print(f"cols statistics {cin} -> {cout}, {d} x {h} x {w}", flush=True)
+    hip, p = ops.hip, ops.hip.ptr
+    x, wt, sx, sw, bias, res, gb = _operands(cin, cout, d, h, w, cin + cout + w)
+    res, gb = res if with_res else None, gb if with_bias else None
+    head, geo, st = (p(x), p(sx), p(wt), p(sw), p(bias)), (cin, d + 2, h + 2, w + 2, cout), hip.stream(DEV)
+    plain = torch.empty(1, d, h, w, cout, dtype=torch.float16, device=DEV)
+    if with_res:
+        hip.call("h3v_conv3d_i8_residual", *head, p(res), p(plain), 1, *geo, 3, 3, 3, 1, 1, 1, 1, st)
+    else:
+        hip.call("h3v_conv3d_i8", *head, p(plain), 1, *geo, 3, 3, 3, 1, 1, 1, 1, st)
+    out = torch.full_like(plain, float("nan"))
+    ws = torch.full((int(hip.lib().h3v_gn_norm_pack_workspace_floats(d, h, w)),), float("nan"), device=DEV)
+    hip.call("h3v_conv3d_i8_cols", *head, p(res), None, p(out), *geo, 1, 0, 0, 0, 0, 0, 0, p(gb), p(ws), st)
+    torch.cuda.synchronize()
+    assert torch.equal(out, plain)
+    n = (h // 8) * (w // 64)
+    k, flat = d * 32 * n, ws.cpu().numpy()
+    avg, m2, ext = oracle.gn_partials_tiled(plain.cpu().numpy()[0], None if gb is None else gb.cpu().numpy())
+    assert np.array_equal(flat[:k].view(np.uint32), avg.reshape(-1).view(np.uint32))
+    assert np.array_equal(flat[k:2 * k].view(np.uint32), m2.reshape(-1).view(np.uint32))
+    assert np.array_equal(flat[2 * k:2 * k + d * n * cout].view(np.uint32), ext.reshape(-1))
+
+
+@pytest.mark.parametrize("cin,cout,d,h,w,front,border,pack_bias", [
+    (128, 128, 2, 8, 192, 2, (1, 1, 1, 1), False), (256, 256, 1, 16, 320, 2, (0, 1, 0, 1), True),
+    (128, 256, 3, 8, 64, 1, (1, 0, 0, 1), True), (128, 128, 1, 24, 640, 0, (0, 0, 0, 0), False)])
+def test_padded_output_at_other_widths(ops, cin, cout, d, h, w, front, border, pack_bias):
+    """h3v_conv3d_i8_cols: the plain conv's output padded as the downsample reads it, bit for bit."""
+    print(f"cols padded {cin} -> {cout}, {d} x {h} x {w}, front {front}, border {border}", flush=True)
+    hip, p = ops.hip, ops.hip.ptr
+    x, wt, sx, sw, bias, res, rb = _operands(cin, cout, d, h, w, cin + cout + w + front)
+    bias, rb = (None, rb) if pack_bias else (bias, None)
+    head, geo, st = (p(x), p(sx), p(wt), p(sw), p(bias)), (cin, d + 2, h + 2, w + 2, cout), hip.stream(DEV)
+    y = torch.empty(1, d, h, w, cout, dtype=torch.float16, device=DEV)
+    hip.call("h3v_conv3d_i8", *head, p(y), 1, *geo, 3, 3, 3, 1, 1, 1, 1, st)
+    v = (res.float() + (y.float() + rb.float())).half() if pack_bias else res + y
+    top, bottom, left, right = border
+    rows = [1] * top + list(range(h)) + [h - 2] * bottom
+    cols = [1] * left + list(range(w)) + [w - 2] * right
+    want = v[:, :, rows][:, :, :, cols]
+    out = torch.full((1, d + front, h + top + bottom, w + left + right, cout), 7.5, dtype=torch.float16, device=DEV)
+    hip.call("h3v_conv3d_i8_cols", *head, p(res), p(rb), p(out), *geo, 1, 1, front, *border, None, None, st)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, front:], want)
+    assert bool((out[:, :front] == 7.5).all())     # the frames in front are the caller's
+
+
+def test_cols_refuses_other_calls(ops):
+    z = torch.zeros(64, device=DEV)
+    p, geo = ops.hip.ptr(z), (128, 4, 10, 66, 128)
+
+    def call(geometry=geo, res=None, rb=None, padded=0, front=0, border=(0, 0, 0, 0), ws=p):
+        ops.hip.call("h3v_conv3d_i8_cols", p, p, p, p, None, res, rb, p, *geometry, 1, padded, front, *border, None, ws,
+                     ops.hip.stream(DEV))
+    for match, kwargs in (("multiple of 64", {"geometry": (128, 4, 10, 98, 128)}),
+                          ("multiple of 8", {"geometry": (128, 4, 14, 66, 128)}),
+                          ("Cin % 128", {"geometry": (64, 4, 10, 66, 128)}),
+                          ("128 or 256", {"geometry": (128, 4, 10, 66, 384)}),
+                          ("either", {"padded": 1}), ("either", {"ws": None}),
+                          ("needs a residual", {"rb": p}), ("alias", {"res": p}),
+                          ("front", {"padded": 1, "ws": None, "front": 17}),
+                          ("border", {"padded": 1, "ws": None, "border": (0, 2, 0, 0)})):
+        with pytest.raises(ValueError, match=match):
+            call(**kwargs)
 
 
 @pytest.mark.parametrize("b,cin,cout,d,h,w", [(1, 64, 128, 3, 120, 192), (1, 128, 128, 2, 64, 640), (1, 256, 256, 3, 40, 320),
