@@ -1574,6 +1574,186 @@ __global__ __launch_bounds__(512) void gemm_i8_pingpong(GemmParams p) {
     }
 }
 
+// Implicit-GEMM convolution on BM x 256 x 128 tiles (BM 256 or 192) with the ping-pong schedule of
+// gemm_i8_pingpong: int8 (Dequant, Int32) or fp16 operands (F16Bias, F32Part with a K split; C and K then count
+// bytes).  Group g owns the rows BM / 2 * g ... of the tile, wave s of a group 64 columns; group 1 moves the
+// activation rows, whose K position runs along with the issues (kd, kh, kw, c0), group 0 the weight rows.  K is
+// long here (18 to 432 steps), so the epilogue is the one of the other tiled kernels, after the groups' barriers
+// have met.  Against gemm_i8_mfma on the same tiles (us, bitwise equal): fp16 256 -> 256 at 9 x 120 x 160 529.7 ->
+// 502.4, 512 -> 512 at 5 x 60 x 80 259.2 -> 255.1, 4 x 1024 -> 1024 at 5 x 16 x 16 (split) 247.2 -> 239.7; int8 256 ->
+// 256 at 17 x 120 x 160 491.6 -> 473.4.
+template <int BM, Epi EP>
+__global__ __launch_bounds__(512) void conv_pingpong(GemmParams p) {
+    constexpr int BN = 256, BK = 128, FM = BM / 64, FN = 2, NSA = 3, NSB = 2;
+    constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK, B_RING = NSA * A_BYTES, RING = B_RING + NSB * B_BYTES;
+    constexpr int PA = BM / 32, PB = BN / 32;                 // DMA instructions per wave and stage (4 waves each)
+    static_assert((BM == 256 || BM == 192) && RING <= 163840, "tile");
+
+    extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar)
+    const int grp = wave >> 2, sw4 = wave & 3;
+
+    int tm, tn;
+    grouped_tile(xcd_remap(blockIdx.x, gridDim.x), p.tiles_m, p.tiles_n, 8, tm, tn);
+    if (p.conv_tpf > 0) {   // one row block for every frame consecutively, as in gemm_i8_mfma
+        const int nf = p.tiles_m / p.conv_tpf;
+        tm = (tm % nf) * p.conv_tpf + tm / nf;
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+
+    // K blocks of this workgroup (a split's share of every depth tap), as in gemm_i8_mfma
+    constexpr bool SPLIT = EP == Epi::F32Part;
+    const int nsplit = SPLIT && p.k_splits > 1 ? p.k_splits : 1;
+    const int third = p.KH * p.KW * p.C / BK, ntap = p.K / BK / third;
+    const int tap0 = conv_first_kblock(p, m0, BM, BK) / third;
+    const int per = (third + nsplit - 1) / nsplit;
+    const int kin = (int)blockIdx.y * per;
+    const int mine = third - kin < per ? third - kin : per;   // may be <= 0 in the last splits
+    const int nk = mine > 0 ? (ntap - tap0) * mine : 0;
+
+    int ck_kd = tap0, a_left = mine, b_blk = tap0 * third + kin, b_left = mine;
+    const int tap_in = kin * BK / p.C, c_in = kin * BK - tap_in * p.C, kh_in = tap_in / p.KW, kw_in = tap_in - kh_in * p.KW;
+    int ck_kh = kh_in, ck_kw = kw_in, ck_c0 = c_in;
+
+    const int lrow = lane >> 3, lslot = lane & 7;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        grp ? __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, (int)p.a_bytes, kRsrcWord3)
+            : __builtin_amdgcn_make_buffer_rsrc((void*)p.b, 0, (int)p.b_bytes, kRsrcWord3);
+    uint32_t doff[PB];                                        // PA <= PB
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+        const int r = (sw4 * (grp ? PA : PB) + j) * 8 + lrow;
+        int64_t base;
+        if (grp) {
+            const int m = m0 + r < p.M ? m0 + r : p.M - 1;
+            base = conv_row_offset(p, m);
+        } else {
+            base = (int64_t)(n0 + r < p.N ? n0 + r : p.N - 1) * p.K;
+        }
+        doff[j] = (uint32_t)(base + ((lslot ^ swz<BK>(r)) << 4));
+    }
+    // the next stage of this group's operand, strictly in order (k counts the stages)
+    auto issue = [&](int k) {
+        if (grp) {
+            const uint32_t off = (uint32_t)((((int64_t)ck_kd * p.Hp + ck_kh) * p.Wp + ck_kw) * p.C + ck_c0);
+            ck_c0 += BK;
+            if (ck_c0 == p.C) {
+                ck_c0 = 0;
+                if (++ck_kw == p.KW) {
+                    ck_kw = 0;
+                    if (++ck_kh == p.KH && !SPLIT) {
+                        ck_kh = 0;
+                        ++ck_kd;
+                    }
+                }
+            }
+            if (SPLIT && --a_left == 0) {
+                a_left = mine;
+                ++ck_kd;
+                ck_kh = kh_in;
+                ck_kw = kw_in;
+                ck_c0 = c_in;
+            }
+            int8_t* dst = smem + (k % NSA) * A_BYTES + sw4 * PA * 1024;
+#pragma unroll
+            for (int j = 0; j < PA; ++j) lds_dma16(rsrc, doff[j], off, dst + j * 1024);
+        } else {
+            const uint32_t off = (uint32_t)(SPLIT ? b_blk++ : b_blk + k) * BK;
+            if (SPLIT && --b_left == 0) {
+                b_left = mine;
+                b_blk += third - mine;
+            }
+            int8_t* dst = smem + B_RING + (k & 1) * B_BYTES + sw4 * PB * 1024;
+#pragma unroll
+            for (int j = 0; j < PB; ++j) lds_dma16(rsrc, doff[j], off, dst + j * 1024);
+        }
+    };
+
+    using Acc = std::conditional_t<kF16Ops<EP>, f32x16, v16i>;
+    Acc acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = Acc{};
+
+    const int frow = lane & 31, fhi = lane >> 5;
+    v4i fa[4][FM], fb[4][FN];   // [ks][block]
+    auto load_frags = [&](int k) {
+        const int8_t* sa = smem + (k % NSA) * A_BYTES;
+        const int8_t* sb = smem + B_RING + (k & 1) * B_BYTES;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int kc = fhi + 2 * ks;
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                const int r = grp * (BM / 2) + i * 32 + frow;
+                fa[ks][i] = *reinterpret_cast<const v4i*>(sa + r * BK + ((kc ^ swz<BK>(r)) << 4));
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int r = sw4 * 64 + j * 32 + frow;
+                fb[ks][j] = *reinterpret_cast<const v4i*>(sb + r * BK + ((kc ^ swz<BK>(r)) << 4));
+            }
+        }
+    };
+    if (nk > 0) {
+        // prologue: weights 0, 1 by group 0; activations 0, 1, 2 by group 1; stage 0 lands before the first barrier
+        issue(0);
+        if (nk > 1) issue(1);
+        if (grp == 0) {
+            if (nk > 1) wait_vmcnt<PB>();
+            else wait_vmcnt<0>();
+        } else {
+            if (nk > 2) { issue(2); wait_vmcnt<2 * PA>(); }
+            else if (nk > 1) wait_vmcnt<PA>();
+            else wait_vmcnt<0>();
+        }
+        lds_barrier();
+        if (grp == 1) lds_barrier();                          // group 1 runs one phase behind
+        __builtin_amdgcn_sched_barrier(0);
+        for (int k = 0; k < nk; ++k) {
+            // load phase of step k
+            load_frags(k);
+            if (k >= 1) {
+                if (grp == 0) { if (k + 1 < nk) issue(k + 1); }
+                else { if (k + 2 < nk) issue(k + 2); }
+            }
+            if (grp == 1 && k + 1 < nk) {                     // activations of step k + 1 land before group 0 reads them
+                if (k + 2 < nk) wait_vmcnt<PA>();
+                else wait_vmcnt<0>();
+            }
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            // MFMA phase of step k
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) {
+                        if constexpr (kF16Ops<EP>)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, fb[ks][j]),
+                                                                              __builtin_bit_cast(half8, fa[ks][i]),
+                                                                              acc[i][j], 0, 0, 0);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[ks][j], fa[ks][i], acc[i][j], 0, 0, 0);
+                    }
+            __builtin_amdgcn_sched_barrier(0);
+            if (grp == 0) {
+                if (k + 1 < nk) wait_vmcnt<0>();              // weights of step k + 1
+                lds_barrier();
+            } else if (k + 1 < nk) {
+                lds_barrier();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    write_tile<BM, BN, 2, 4, RING, EP>(p, acc, smem, m0, n0, tn);
+}
+
 // Window row pitch in pixels of conv3_halo_i8 for tiles TW pixels wide: TW + 2 rounded up to 16 (the
 // plain swizzle works on 16-pixel groups) or, in the strided-pixel variant, to 8 (whole 256-byte lines).
 constexpr int halo_hpl(int tw, bool sp) { return sp ? (tw + 2 + 7) / 8 * 8 : (tw + 2 + 15) / 16 * 16; }
@@ -2024,6 +2204,37 @@ __global__ __launch_bounds__(256) void gemm_i8_generic(GemmParams p) {
     }
 }
 
+// Convolution through conv_pingpong: C bytes a multiple of 128.
+template <int BM, Epi EP>
+int launch_conv_pingpong(GemmParams p, hipStream_t stream, const char* what) {
+    p.tiles_m = (p.M + BM - 1) / BM;
+    p.tiles_n = (p.N + 255) / 256;
+    p.vec_epi = (p.sw == nullptr || aligned(p.sw, 16)) && (p.bias == nullptr || aligned(p.bias, 8)) && p.N % 4 == 0;
+    p.vec_out = aligned(p.out, 16) && (p.res == nullptr || aligned(p.res, 16)) && p.ldo % 8 == 0;
+    const int64_t hw = (int64_t)p.Ho * p.Wo;
+    p.conv_tpf = hw % BM == 0 ? (int)(hw / BM) : 0;
+    const int64_t grid = (int64_t)p.tiles_m * p.tiles_n;
+    if (grid > 0x7fffffff) return fail(H3V_EINVAL, "%s: too many tiles", what);
+    const int64_t a_bytes = (int64_t)(p.M / ((int64_t)p.Do * hw)) * p.Dp * p.Hp * p.Wp * p.C, b_bytes = (int64_t)p.N * p.K;
+    if (a_bytes >= ((int64_t)1 << 32) || b_bytes >= ((int64_t)1 << 32))
+        return fail(H3V_EINVAL, "%s: an operand exceeds 4 GiB (%lld, %lld bytes)", what, (long long)a_bytes,
+                    (long long)b_bytes);
+    p.a_bytes = (uint32_t)a_bytes;
+    p.b_bytes = (uint32_t)b_bytes;
+    if (p.gn_avg != nullptr) return fail(H3V_EINVAL, "%s: no statistics epilogue for this tile", what);
+    constexpr size_t lds = (size_t)(3 * BM + 2 * 256) * 128;
+    auto kernel = &conv_pingpong<BM, EP>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (attr != hipSuccess) return fail(H3V_ELAUNCH, "%s: cannot reserve %zu bytes of LDS: %s", what, lds,
+                                        hipGetErrorString(attr));
+    const int splits = p.k_splits > 1 ? p.k_splits : 1;
+    if ((p.K / 128) % splits != 0 || (splits > 1 && EP != Epi::F32Part))
+        return fail(H3V_EINVAL, "%s: %d K splits do not divide %d K blocks", what, splits, p.K / 128);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid, (unsigned)splits), dim3(512), lds, stream, p);
+    return launch_status(what);
+}
+
 template <int BM, int BN, int BK, int WGM, int WGN, int NSA, int NSB, AMode AM, Epi EP>
 int launch_tiled(GemmParams p, hipStream_t stream, const char* what) {
     int ncols = (EP == Epi::SwiGLU) ? 2 * p.N : p.N;
@@ -2417,7 +2628,7 @@ int run_conv(GemmParams p, hipStream_t stream, const char* what) {
     if (halo_tiles >= 128 && cols_conv_fits(p)) return launch_cols<EP>(p, stream, what);
     if (al && p.C % 128 == 0) {
         if (p.N <= 128) return launch_tiled<512, 128, 128, 4, 2, 2, 2, AMode::Conv, EP>(p, stream, what);
-        return launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, EP>(p, stream, what);
+        return launch_conv_pingpong<256, EP>(p, stream, what);
     }
     if (al && p.C % 64 == 0) {
         if (p.N <= 128) return launch_tiled<512, 128, 64, 4, 2, 4, 4, AMode::Conv, EP>(p, stream, what);
@@ -2684,9 +2895,9 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
         q.res = nullptr;
         q.k_splits = plan.splits;
         if (plan.kind == F16Kind::Tiled256x256)
-            rc = launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
+            rc = launch_conv_pingpong<256, Epi::F32Part>(q, stream, what);
         else if (plan.kind == F16Kind::Tiled192x256)
-            rc = launch_tiled<192, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
+            rc = launch_conv_pingpong<192, Epi::F32Part>(q, stream, what);
         else
             rc = launch_tiled<256, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F32Part>(q, stream, what);
         if (rc) return rc;
@@ -2698,8 +2909,8 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
     switch (plan.kind) {
         case F16Kind::Tiled512x128: return launch_tiled<512, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x128: return launch_tiled<256, 128, 128, 4, 2, 2, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
-        case F16Kind::Tiled256x256: return launch_tiled<256, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
-        case F16Kind::Tiled192x256: return launch_tiled<192, 256, 128, 2, 4, 3, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
+        case F16Kind::Tiled256x256: return launch_conv_pingpong<256, Epi::F16Bias>(p, stream, what);
+        case F16Kind::Tiled192x256: return launch_conv_pingpong<192, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x128k64: return launch_tiled<256, 128, 64, 4, 2, 4, 4, AMode::Conv, Epi::F16Bias>(p, stream, what);
         case F16Kind::Tiled256x128k64r3: return launch_tiled<256, 128, 64, 4, 2, 3, 2, AMode::Conv, Epi::F16Bias>(p, stream, what);
         default: return launch_tiled<256, 256, 64, 2, 4, 4, 4, AMode::Conv, Epi::F16Bias>(p, stream, what);
