@@ -133,16 +133,40 @@ __device__ __forceinline__ void conv_row_frame(const GemmParams& p, int m, int& 
 // Causal-zero skip: the fused producer writes two zero frames in front of the
 // input, so for output frame t the taps kd < 2 - t multiply zeros.  A tile may
 // skip them only if every row in it allows it, i.e. for the largest frame.
-__device__ __forceinline__ int conv_first_kblock(const GemmParams& p, int m0, int bm, int bk) {
+// Returns the first depth tap of the tile.
+__device__ __forceinline__ int conv_first_tap(const GemmParams& p, int m0, int bm) {
     if (!p.causal_skip) return 0;
     int last = m0 + bm - 1 < p.M - 1 ? m0 + bm - 1 : p.M - 1;
     int b0, t0, b1, t1;
     conv_row_frame(p, m0, b0, t0);
     conv_row_frame(p, last, b1, t1);
     int tmax = (b0 != b1) ? p.Do - 1 : t1;
-    int skip = 2 - tmax;
-    if (skip <= 0) return 0;
-    return skip * p.KH * p.KW * p.C / bk;
+    return tmax < 2 ? 2 - tmax : 0;
+}
+
+// K blocks of a workgroup of the tiled kernels, BK bytes each: all of them past the causal-zero depth taps of a
+// conv tile's first frames.  With a K split the K blocks of one depth tap are `third`, and split blockIdx.y of
+// k_splits takes the `mine` blocks from kin on of every depth tap, so the splits stay even when depth taps are
+// skipped, and add up the same numbers.
+struct KRange {
+    int third, tap0, kin, mine, nk;
+};
+template <bool CONV, bool SPLIT>
+__device__ __forceinline__ KRange k_range(const GemmParams& p, int m0, int bm, int bk) {
+    KRange r;
+    r.third = CONV ? p.KH * p.KW * p.C / bk : p.K / bk;
+    r.tap0 = CONV ? conv_first_tap(p, m0, bm) : 0;
+    r.kin = 0;
+    r.mine = r.third;
+    r.nk = p.K / bk - r.tap0 * r.third;
+    if constexpr (SPLIT) {
+        const int nsplit = p.k_splits > 1 ? p.k_splits : 1;
+        const int per = (r.third + nsplit - 1) / nsplit;
+        r.kin = (int)blockIdx.y * per;
+        r.mine = r.third - r.kin < per ? r.third - r.kin : per;   // may be <= 0 in the last splits
+        r.nk = r.mine > 0 ? (p.K / bk / r.third - r.tap0) * r.mine : 0;
+    }
+    return r;
 }
 
 __device__ __forceinline__ float g1_value(int32_t acc, float sx, float sw, const uint16_t* bias, int col) {
@@ -969,34 +993,21 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_i8_mfma(GemmParams p) {
         boff[j] = (uint32_t)((int64_t)wrow * p.K + ((lslot ^ swz<BK>(r)) << 4));
     }
 
-    // K blocks of this workgroup: all of them past the causal-zero depth taps of a conv tile's first frames.  With a
-    // K split (F32Part): the K blocks of one depth tap are `third`, and split blockIdx.y of k_splits takes the blocks
-    // from kin on of every depth tap, `mine` of each, so the splits stay even when depth taps are skipped, and add up
-    // the same numbers.
     constexpr bool SPLIT = EP == Epi::F32Part;
-    const int nsplit = SPLIT && p.k_splits > 1 ? p.k_splits : 1;
-    int third = p.K / BK, ntap = 1, tap0 = 0;                 // depth taps and the first one that is not skipped
-    if constexpr (AM == AMode::Conv) {
-        third = p.KH * p.KW * p.C / BK;
-        ntap = p.K / BK / third;
-        tap0 = conv_first_kblock(p, m0, BM, BK) / third;
-    }
-    const int per = (third + nsplit - 1) / nsplit;
-    const int kin = (int)blockIdx.y * per;
-    const int mine = third - kin < per ? third - kin : per;   // may be <= 0 in the last splits
-    const int nk = mine > 0 ? (ntap - tap0) * mine : 0;
+    const KRange kr = k_range<AM == AMode::Conv, SPLIT>(p, m0, BM, BK);
+    const int third = kr.third, kin = kr.kin, mine = kr.mine, nk = kr.nk;
 
     // A and B stages are issued strictly in order, so their k positions are kept running: no integer division
     // in the loop.  The conv's A position is (kd, kh, kw, c0).
-    int ck_kd = tap0, ck_kh = 0, ck_kw = 0, ck_c0 = 0, a_left = mine;
-    if constexpr (AM == AMode::Conv) {
+    int ck_kd = kr.tap0, ck_kh = 0, ck_kw = 0, ck_c0 = 0, a_left = mine;
+    if constexpr (AM == AMode::Conv && SPLIT) {
         const int tap = kin * BK / p.C;
         ck_c0 = kin * BK - tap * p.C;
         ck_kh = tap / p.KW;
         ck_kw = tap - ck_kh * p.KW;
     }
     const int kh_in = ck_kh, kw_in = ck_kw, c_in = ck_c0;
-    int b_blk = tap0 * third + kin, b_left = mine;
+    int b_blk = kr.tap0 * third + kin, b_left = mine;
     auto issue_a = [&](int it) {
         int8_t* sa = smem + (it % NSA) * A_BYTES;
         int64_t koff;
@@ -1604,19 +1615,18 @@ __global__ __launch_bounds__(512) void conv_pingpong(GemmParams p) {
     }
     const int m0 = tm * BM, n0 = tn * BN;
 
-    // K blocks of this workgroup (a split's share of every depth tap), as in gemm_i8_mfma
     constexpr bool SPLIT = EP == Epi::F32Part;
-    const int nsplit = SPLIT && p.k_splits > 1 ? p.k_splits : 1;
-    const int third = p.KH * p.KW * p.C / BK, ntap = p.K / BK / third;
-    const int tap0 = conv_first_kblock(p, m0, BM, BK) / third;
-    const int per = (third + nsplit - 1) / nsplit;
-    const int kin = (int)blockIdx.y * per;
-    const int mine = third - kin < per ? third - kin : per;   // may be <= 0 in the last splits
-    const int nk = mine > 0 ? (ntap - tap0) * mine : 0;
-
-    int ck_kd = tap0, a_left = mine, b_blk = tap0 * third + kin, b_left = mine;
-    const int tap_in = kin * BK / p.C, c_in = kin * BK - tap_in * p.C, kh_in = tap_in / p.KW, kw_in = tap_in - kh_in * p.KW;
-    int ck_kh = kh_in, ck_kw = kw_in, ck_c0 = c_in;
+    const KRange kr = k_range<true, SPLIT>(p, m0, BM, BK);
+    const int third = kr.third, mine = kr.mine, nk = kr.nk;
+    int ck_kd = kr.tap0, ck_kh = 0, ck_kw = 0, ck_c0 = 0, a_left = mine;
+    if constexpr (SPLIT) {
+        const int tap = kr.kin * BK / p.C;
+        ck_c0 = kr.kin * BK - tap * p.C;
+        ck_kh = tap / p.KW;
+        ck_kw = tap - ck_kh * p.KW;
+    }
+    const int kh_in = ck_kh, kw_in = ck_kw, c_in = ck_c0;
+    int b_blk = kr.tap0 * third + kr.kin, b_left = mine;
 
     const int lrow = lane >> 3, lslot = lane & 7;
     const __amdgpu_buffer_rsrc_t rsrc =
