@@ -74,6 +74,7 @@ namespace {
 constexpr int kGroups = 32;
 constexpr int kChunk = 256;
 constexpr int kNT = 256;
+constexpr int kMergeInline = 20;   // chunks per frame up to which norm_pack_f16 merges them itself
 constexpr int kF16Unroll = 4;   // vectors of 8 channels a thread of norm_pack_f16 has in flight
 constexpr int kMaxC = 256;
 constexpr float kShortcutFloor = 0.5f;
@@ -740,15 +741,23 @@ __global__ __launch_bounds__(64) void gn_stats_merge(const float* __restrict__ p
 // in steps that are a multiple of C/8, so each keeps one 8-channel slice.  A
 // thread loads four vectors before it works on any (with one in flight at a time
 // a block waited for memory in every step), and gridDim.y blocks share a row
-// where the rows alone are too few (f16_row_blocks).  Per call, one row per block
+// where the rows alone are too few (f16_row_blocks).  MERGE: frames of at most
+// kMergeInline chunks have no merge launch; 32 threads of each block merge the
+// groups' partials in chunk order themselves, as gn_merge_group does (up to about
+// 1 us a block, eight of which share a CU, against a launch of 3 to 5 us and the
+// host's time for it: statistics and pack of 512 x 1 x 32 x 32 14.5 -> 12.8 us,
+// 4 x 1024 x 5 x 16 x 16 26.6 -> 24.5), unless very many blocks would (4 x 256 x 9 x
+// 64 x 64, 16 chunks in 5808 blocks: 62.0 / 62.5).  Per call, one row per block
 // and one load at a time against this: 1024 x 5 x 30 x 40 29.0 -> 12.3 us, 512 x 5 x
 // 60 x 80 32.5 -> 17.0, 256 x 9 x 120 x 160 50.0 -> 40.6 (4.4 TB/s); bitwise equal.
-template <int C, bool PRE_BIAS>
+template <int C, bool PRE_BIAS, bool MERGE>
 __global__ __launch_bounds__(kNT) void norm_pack_f16(const uint16_t* __restrict__ x,
                                                      const uint16_t* __restrict__ pre_bias,
                                                      const uint16_t* __restrict__ gamma,
-                                                     const uint16_t* __restrict__ beta, const float* __restrict__ stats,
-                                                     int d, int h, int w, uint16_t* __restrict__ y) {
+                                                     const uint16_t* __restrict__ beta, float* stats,
+                                                     const float* __restrict__ part_avg,
+                                                     const float* __restrict__ part_m2, int nchunk, float eps, int d,
+                                                     int h, int w, uint16_t* __restrict__ y) {
     constexpr int CG = C / kGroups;
     constexpr int TPP = C / 8;
     constexpr int NG = 8 / CG > 1 ? 8 / CG : 1;   // groups touched by one 8-channel slice
@@ -775,10 +784,52 @@ __global__ __launch_bounds__(kNT) void norm_pack_f16(const uint16_t* __restrict_
     const int frame = b * d + t;
     const int g0 = cv * 8 / CG;
     float mean[NG], rstd[NG];
+    if constexpr (MERGE) {
+        __shared__ float pa[kGroups * (kMergeInline + 1)], pm[kGroups * (kMergeInline + 1)];   // rows of odd pitch
+        __shared__ float ms[kGroups][2];
+        const int64_t first = (int64_t)frame * kGroups * nchunk;
+        for (int i = threadIdx.x; i < kGroups * nchunk; i += kNT) {
+            const int at = i / nchunk * (kMergeInline + 1) + i % nchunk;
+            pa[at] = part_avg[first + i];
+            pm[at] = part_m2[first + i];
+        }
+        __syncthreads();
+        if (threadIdx.x < kGroups) {
+            const float* const a = pa + threadIdx.x * (kMergeInline + 1);
+            const float* const m = pm + threadIdx.x * (kMergeInline + 1);
+            constexpr int CHUNK = GnGeom<C>::CHUNK;
+            const int hw = h * w;
+            const float total = (float)(hw * CG);
+            auto weight = [&](int j) { return (float)((hw - j * CHUNK < CHUNK ? hw - j * CHUNK : CHUNK) * CG); };
+            float san = 0.0f, sv = 0.0f;
+            for (int j = 0; j < nchunk; ++j) san = san + a[j] * weight(j);
+            const float mn = san / total;
+            for (int j = 0; j < nchunk; ++j) {
+                const float dl = a[j] - mn;
+                sv = sv + (m[j] + (weight(j) * dl) * dl);
+            }
+            float var = sv / total;
+            if (var < 0.0f) var = 0.0f;
+            const float rs = rsqrt_rn(var + eps);
+            ms[threadIdx.x][0] = mn;
+            ms[threadIdx.x][1] = rs;
+            if (ii == 0 && blockIdx.y == 0) {
+                stats[(frame * kGroups + threadIdx.x) * 2] = mn;
+                stats[(frame * kGroups + threadIdx.x) * 2 + 1] = rs;
+            }
+        }
+        __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NG; ++k) {
-        mean[k] = stats[(frame * kGroups + g0 + k) * 2];
-        rstd[k] = stats[(frame * kGroups + g0 + k) * 2 + 1];
+        for (int k = 0; k < NG; ++k) {
+            mean[k] = ms[g0 + k][0];
+            rstd[k] = ms[g0 + k][1];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NG; ++k) {
+            mean[k] = stats[(frame * kGroups + g0 + k) * 2];
+            rstd[k] = stats[(frame * kGroups + g0 + k) * 2 + 1];
+        }
     }
     const uint16_t* src = x + ((int64_t)frame * h + reflect(ii - 1, h)) * w * C + cv * 8;
     const int step = gridDim.y * kF16Unroll * kNT;
@@ -822,11 +873,18 @@ void launch_f16(const uint16_t* x, const uint16_t* pre_bias, const uint16_t* gam
     float* part_m2 = ws + (int64_t)frames * nchunk * kGroups;
     hipLaunchKernelGGL((gn_stats_partial<C, PB>), dim3(nchunk, frames), dim3(kNT), 0, stream, x, pre_bias, hw, nchunk,
                        part_avg, part_m2);
-    hipLaunchKernelGGL(gn_stats_merge, dim3(kGroups, frames), dim3(64), 0, stream, part_avg, part_m2, hw, nchunk, chunk,
-                       C, eps, stats);
     const int rows = batch * (d + 2) * (h + 2);
-    hipLaunchKernelGGL((norm_pack_f16<C, PB>), dim3(rows, f16_row_blocks(rows, (w + 2) * (C / 8))), dim3(kNT), 0, stream,
-                       x, pre_bias, gamma, beta, stats, d, h, w, y);
+    const dim3 grid(rows, f16_row_blocks(rows, (w + 2) * (C / 8)));
+    const bool merge = nchunk <= kMergeInline && (int64_t)nchunk * grid.x * grid.y <= 40000;
+    if (!merge)
+        hipLaunchKernelGGL(gn_stats_merge, dim3(kGroups, frames), dim3(64), 0, stream, part_avg, part_m2, hw, nchunk,
+                           chunk, C, eps, stats);
+    if (merge)
+        hipLaunchKernelGGL((norm_pack_f16<C, PB, true>), grid, dim3(kNT), 0, stream, x, pre_bias, gamma, beta, stats,
+                           part_avg, part_m2, nchunk, eps, d, h, w, y);
+    else
+        hipLaunchKernelGGL((norm_pack_f16<C, PB, false>), grid, dim3(kNT), 0, stream, x, pre_bias, gamma, beta, stats,
+                           part_avg, part_m2, nchunk, eps, d, h, w, y);
 }
 
 
