@@ -77,7 +77,8 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
 // QS sets of 32 queries per wave, NW waves (8 or 4; 32 * NW * QS queries per workgroup); every K and V^T
 // fragment read from LDS feeds the MFMAs of all QS sets (two sets: 233 VGPRs, 2 waves per SIMD; one: 150, 3
 // waves).  Waves 0-3 move each K / V block into LDS for all 8 (half the per-query load and transpose work of
-// 4-wave workgroups).  Every query goes through the same operations in the same order whatever QS and NW are.
+// 4-wave workgroups).  Every query goes through the same operations in the same order whatever QS and NW are, but
+// for the blocks that move a reference maximum, which the queries of a wave do together.
 // PART: one split of the keys, its unnormalised outputs and (m_ref, sum) pairs to p.part / p.ml (fp32).
 template <int QS, int NW, bool PART>
 __global__ __launch_bounds__(64 * NW) void fmha_d64(AttnParams p) {
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(64 * NW) void fmha_d64(AttnParams p) {
         oacc[qs][0] = f32x16{};
         oacc[qs][1] = f32x16{};
         m_ref[qs] = -__builtin_inff();
-        mc[qs] = -__builtin_inff();
+        mc[qs] = PART ? 0.0f : -__builtin_inff();
         l_run[qs] = 0.0f;
     }
     const float thr = kLazy / p.c;   // raw-score margin of the lazy maximum
@@ -246,9 +247,16 @@ __global__ __launch_bounds__(64 * NW) void fmha_d64(AttnParams p) {
 #pragma unroll
             for (int qs = 0; qs < QS; ++qs) {
                 const float m_new = __builtin_fmaxf(m_ref[qs], mblk[qs]);
-                const float alpha = __builtin_amdgcn_exp2f((m_ref[qs] - m_new) * p.c);   // 0 from -inf, 1 if unmoved
+                float alpha = __builtin_amdgcn_exp2f((m_ref[qs] - m_new) * p.c);   // 0 from -inf, 1 if unmoved
                 m_ref[qs] = m_new;
                 mc[qs] = m_new * p.c;
+                if constexpr (PART) {
+                    // a split whose scores are all -inf so far has weights of 0 (another split has the others)
+                    if (m_new == -__builtin_inff()) {
+                        alpha = 1.0f;
+                        mc[qs] = 0.0f;
+                    }
+                }
                 l_run[qs] *= alpha;
 #pragma unroll
                 for (int db = 0; db < 2; ++db)

@@ -174,6 +174,25 @@ def test_attention_key_splits_carry_large_scores(ops, oracle):
     _check(ops, oracle, q[:, :, :2], k[:, :, :2], v[:, :, :2].contiguous(), out[:, :, :2], queries)
 
 
+@pytest.mark.parametrize("first,last", [(1024, 2049), (512, 1600)])
+def test_attention_key_splits_without_a_finite_score(ops, first, last):
+    """Keys of minus infinite score over whole splits weigh nothing, in the split queries as in the others."""
+    b, n, h = 2, 2049, 32
+    q, k, v, qd, kd, vd = _qkv(b, n, h, seed=23)
+    qd, kd = qd.clone(), kd.clone()
+    qd[..., 0] = qd[..., 0].abs() + 0.1
+    kd[:, first:last, :, 0] = -float("inf")
+    with torch.inference_mode():
+        out = ops.decoder_fused_qk_rope.attention_d64(qd, kd, vd, 0.125)
+    torch.cuda.synchronize()
+    keep = [t for t in range(n) if not first <= t < last]
+    for i in (0, 2000, 2047, 2048):
+        qs, ks, vs = (x.double().cpu().transpose(1, 2) for x in (qd[:, i:i + 1], kd[:, keep], vd[:, keep]))
+        want = torch.softmax(qs @ ks.transpose(2, 3).contiguous() * 0.125, dim=-1) @ vs
+        err = (out[:, i:i + 1].double().cpu().transpose(1, 2) - want).abs()
+        assert bool((err <= 2e-3 + 4e-3 * want.abs()).all())
+
+
 def test_attention_workspace_is_required_for_splits(ops):
     b, n, h = 4, 1025, 32
     x = torch.zeros(b, n, h, 64, dtype=torch.float16, device=DEV)
