@@ -2360,7 +2360,7 @@ int f16_splits(int64_t tiles, int kblocks) {
 // four 32-row blocks share a weight fragment), a 256 x 128 one half and 15%; a split's partial sums are written and
 // read at about 5 TB/s, and the second kernel takes 6 us.  Up to three rounds count whole; over more, the tiles'
 // ends drift apart.  `active` is the share of K a tile runs (a causal conv of one frame skips two thirds).
-// Start against now (us, causal): 4 x 512 -> 512 at 5 x 32 x 32 (160 window tiles against 214 of 192 rows) 238.9 ->
+// Before and now (us, causal): 4 x 512 -> 512 at 5 x 32 x 32 (160 window tiles against 214 of 192 rows) 238.9 ->
 // 225.8, one clip (40 window tiles, six splits) 213.4 -> 78.6, 512 -> 512 at 5 x 60 x 80 (188 tiles of 256 rows,
 // 250 of 192) 284.8 -> 244.2, 512 -> 512 at 1 x 32 x 32 73.8 -> 25.0.
 struct WidePlan {
@@ -2880,7 +2880,8 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
     p.causal_skip = (causal_skip && kd == 3 && sd == 1) ? 1 : 0;
     H3V_REQUIRE(cin % 32 == 0 && aligned(x, 16) && aligned(w, 16),
                 "%s: requires Cin %% 32 == 0 and 16-byte aligned x and w (got Cin %d)", what, cin);
-    const F16Plan plan = plan_conv_f16(p, may_split);
+    // the reduction of the splits stores 8-byte pieces
+    const F16Plan plan = plan_conv_f16(p, may_split && aligned(out, 8) && (residual == nullptr || aligned(residual, 8)));
     switch (plan.kind) {
         case F16Kind::Cols: return launch_cols<Epi::F16Bias, 2>(p, stream, what);
         case F16Kind::Halo256: return launch_halo<256, Epi::F16Bias, 2>(p, stream, what);
@@ -2897,8 +2898,6 @@ static int conv3d_f16_common(const uint16_t* x, const uint16_t* w, const uint16_
         H3V_REQUIRE(workspace != nullptr && workspace_floats >= need && aligned(workspace, 16),
                     "%s: this shape splits K %d ways and needs a 16-byte aligned workspace of %lld floats (got %lld)",
                     what, plan.splits, (long long)need, (long long)workspace_floats);
-        H3V_REQUIRE(p.N % 4 == 0 && aligned(out, 8) && (residual == nullptr || aligned(residual, 8)),
-                    "%s: a split reduction needs Cout %% 4 == 0 and 8-byte aligned output and residual", what);
         GemmParams q = p;
         q.out = workspace;
         q.bias = nullptr;

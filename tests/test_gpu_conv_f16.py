@@ -194,6 +194,26 @@ def test_conv3d_f16_split_reduction_matches_float64(fc, b, c, d, h, w, cout, cau
                      floats - 1, fc._hip.stream(DEV))
 
 
+@pytest.mark.parametrize("c,d,h,w", [(512, 7, 34, 34), (512, 5, 42, 30)])
+def test_conv3d_f16_residual_between_8_byte_boundaries(fc, c, d, h, w):
+    """The reduction of the splits stores 8-byte pieces: other residuals run the convolution unsplit."""
+    print(f"conv3d_f16 unaligned residual C={c} D={d} {h}x{w}", flush=True)
+    assert int(fc._hip.lib().h3v_conv3d_f16_workspace_floats(1, c, d, h, w, c, 3, 3, 3, 1, 1, 1)) > 0
+    x, wt, bias = _operands(1, c, d, h, w, c, True, seed=c + h, causal_zero=True)
+    xd, wp, bd = x.to(DEV).contiguous(memory_format=torch.channels_last_3d), fc.pack_conv_weight_f16(wt.to(DEV)), bias.to(DEV)
+    shape = (1, d - 2, h - 2, w - 2, c)
+    flat = torch.randn(torch.Size(shape).numel() + 1, generator=torch.Generator().manual_seed(h)).half().to(DEV)
+    rd = flat[1:].view(shape).permute(0, 4, 1, 2, 3)
+    assert rd.data_ptr() % 8 == 2 and rd.is_contiguous(memory_format=torch.channels_last_3d)
+    with torch.inference_mode():
+        fused = fc.conv3d_f16(xd, wp, bd, [3, 3, 3], [1, 1, 1], True, rd)
+    plain = torch.empty_like(fused)
+    fc._hip.call("h3v_conv3d_f16", fc._hip.ptr(xd), fc._hip.ptr(wp), fc._hip.ptr(bd), None, fc._hip.ptr(plain), 1, c, d,
+                 h, w, c, 3, 3, 3, 1, 1, 1, 1, fc._hip.stream(DEV))
+    torch.cuda.synchronize()
+    assert torch.equal(fused, rd + plain)
+
+
 @pytest.mark.parametrize("d,cout", [(18, 32), (10, 48)])
 def test_conv3d_f16_row_tile_choice_sampled_frames(fc, d, cout):
     """Cout <= 128 implicit GEMM at full size: 16 output frames of 64 x 128 (131072 rows) fill whole rounds
