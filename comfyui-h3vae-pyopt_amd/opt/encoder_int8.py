@@ -224,6 +224,7 @@ def _conv3d_from_quantized(qx, activation_scale, qweight, weight_scale, *, confi
             _hip.call("h3v_conv3d_i8_gn", *head, _hip.ptr(residual), _hip.ptr(out), *geometry, _hip.ptr(gn_bias),
                       _hip.ptr(gn_workspace), _hip.stream(qx.device))
         else:
+            residual, gn_bias = _aligned16(residual), _aligned16(gn_bias)
             _hip.call("h3v_conv3d_i8_cols", *head, _hip.ptr(residual), None, _hip.ptr(out), *geometry, 0, 0, 0, 0, 0, 0,
                       _hip.ptr(gn_bias), _hip.ptr(gn_workspace), _hip.stream(qx.device))
         return out
@@ -234,6 +235,12 @@ def _conv3d_from_quantized(qx, activation_scale, qweight, weight_scale, *, confi
         return out
     _hip.call("h3v_conv3d_i8_residual", *head, _hip.ptr(residual), _hip.ptr(out), *geometry, _hip.stream(qx.device))
     return out
+
+
+def _aligned16(t):
+    """t, or a copy of it where it is a view that starts between two 16-byte boundaries (the window conv's statistics
+    and padded outputs read 16-byte pieces)."""
+    return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
 
 
 def gn_stats_fits(in_channels: int, out_channels: int, out_d: int, out_h: int, out_w: int, *, batch: int = 1) -> bool:
@@ -293,10 +300,13 @@ def _conv3d_from_quantized_padded(qx, activation_scale, qweight, weight_scale, *
                                       or residual_bias.dtype != torch.float16):
         raise ValueError("residual_bias needs a residual and must be an fp16 vector of the output channels")
     residual_bias = None if residual_bias is None else residual_bias.contiguous()
+    cols = b == 1 and wo > 128 and wo != 256 and wo % 64 == 0
+    if cols:
+        residual, residual_bias = _aligned16(residual), _aligned16(residual_bias)
     head = (_hip.ptr(qx), _hip.ptr(activation_scale), _hip.ptr(qweight), _hip.ptr(weight_scale), _hip.ptr(bias),
             _hip.ptr(residual), _hip.ptr(residual_bias), _hip.ptr(out))
     border = (int(front), top, bottom, left, right)
-    if b == 1 and wo > 128 and wo != 256 and wo % 64 == 0:
+    if cols:
         _hip.call("h3v_conv3d_i8_cols", *head, *qx.shape[1:], cout, 1, 1, *border, None, None, _hip.stream(qx.device))
     else:
         _hip.call("h3v_conv3d_i8_residual_padded", *head, *qx.shape, cout, 1, *border, _hip.stream(qx.device))

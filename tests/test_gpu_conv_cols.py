@@ -118,6 +118,37 @@ def test_padded_output_at_other_widths(ops, cin, cout, d, h, w, front, border, p
     assert bool((out[:, :front] == 7.5).all())     # the frames in front are the caller's
 
 
+def _between_boundaries(t):
+    """The same values and strides, starting 2 bytes past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    view = flat[1:].as_strided(t.shape, t.stride(), 1)
+    assert view.copy_(t).data_ptr() % 16 == 2
+    return view
+
+
+@pytest.mark.parametrize("padded", [False, True])
+def test_residual_and_biases_between_16_byte_boundaries(ops, padded):
+    """The Python entries take such views at these widths as they do where the plain conv runs."""
+    print(f"cols unaligned views, padded {padded}", flush=True)
+    e8 = ops.encoder_int8
+    x, wt, sx, sw, bias, res, gb = _operands(128, 128, 6, 64, 192, 5)
+    qx, res = x.permute(0, 4, 1, 2, 3), res.permute(0, 4, 1, 2, 3)
+
+    def run(res, extra):
+        if padded:
+            return e8._conv3d_from_quantized_padded(qx, sx, wt, sw, bias=None, residual=res, residual_bias=extra, front=2,
+                                                    border=(0, 1, 0, 1))
+        ws = torch.zeros(e8.gn_workspace_floats(6, 64, 192), device=DEV)
+        config = e8.Int8Conv3DConfig(128, 128, (3, 3, 3), (1, 1, 1))
+        out = e8._conv3d_from_quantized(qx, sx, wt, sw, config=config, bias=bias, tile_variant="64x64x64",
+                                        causal_prefix_zero=True, residual=res, gn_workspace=ws, gn_bias=extra)
+        return torch.cat([out.flatten().float(), ws[:2 * 6 * 32 * 24]])
+    with torch.inference_mode():
+        want, got = run(res, gb), run(_between_boundaries(res), _between_boundaries(gb))
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
 def test_cols_refuses_other_calls(ops):
     z = torch.zeros(64, device=DEV)
     p, geo = ops.hip.ptr(z), (128, 4, 10, 66, 128)
