@@ -1094,7 +1094,7 @@ def main():
             "in_step": in_step_summary(in_step, "gemm"),
         },
         "roofline_stage0_conv": {
-            "kernel": "conv3_halo_i8<256,Dequant,SP,64> (stage-0 conv C128->128, strided pixels on 64-pixel column blocks, "
+            "kernel": "conv3_halo_i8<0,Dequant,SP,64> (stage-0 conv C128->128, strided pixels on 64-pixel column blocks, "
                       "[1,128,19,258,258] int8, no residual, with the GroupNorm tile statistics of its output)",
             "bound": "mfma",
             "achieved": round(achieved, 1),
