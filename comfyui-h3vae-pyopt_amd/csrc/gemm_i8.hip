@@ -2328,11 +2328,13 @@ bool halo_conv_fits(const GemmParams& p, int es = 1) {
 }
 
 // Whether a stride-1 3x3x3 convolution with ES-byte elements takes the strided-pixel kernel: whole 8-row tiles of
-// 64-pixel column blocks and stages in groups of four (C * ES % 128 == 0).
+// 64-pixel column blocks and stages in groups of four (C * ES % 128 == 0).  Weights of 2 GiB and more, past its
+// 32-bit offsets, stay with the implicit GEMM, which takes up to 4 GiB.
 bool cols_conv_fits(const GemmParams& p, int es = 1) {
     const bool shape = p.KH == 3 && p.KW == 3 && p.K == 27 * p.C && p.SD == 1 && p.SH == 1 && p.SW == 1 &&
                        (p.C * es) % 128 == 0 && p.N % 128 == 0 && p.Wo % 64 == 0 && p.Ho % 8 == 0;
-    return shape && aligned(p.a, 16) && aligned(p.b, 16) && (int64_t)p.Hp * p.Wp * p.C * es * 3 < ((int64_t)1 << 31);
+    return shape && aligned(p.a, 16) && aligned(p.b, 16) && (int64_t)p.Hp * p.Wp * p.C * es * 3 < ((int64_t)1 << 31) &&
+           (int64_t)p.N * p.K * es < ((int64_t)1 << 31);
 }
 
 enum class F16Kind { Cols, Halo256, Halo128, Halo64, Halo32, Tiled512x128, Tiled256x128, Tiled256x256, Tiled192x256,

@@ -243,6 +243,12 @@ def _aligned16(t):
     return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _cols_in_range(in_channels: int, out_channels: int, out_h: int, out_w: int) -> bool:
+    """Whether three padded input frames and the weights stay within the window conv's signed 32-bit byte offsets;
+    larger ones (a 2400 x 2432 image at 128 channels) run as the implicit GEMM, which takes up to 4 GiB."""
+    return 3 * (out_h + 2) * (out_w + 2) * in_channels < 2 ** 31 and 27 * in_channels * out_channels < 2 ** 31
+
+
 def gn_stats_fits(in_channels: int, out_channels: int, out_d: int, out_h: int, out_w: int, *, batch: int = 1) -> bool:
     """Whether ``h3v_conv3d_i8_gn`` or ``h3v_conv3d_i8_cols`` takes a stride-1 3x3x3 conv of this geometry and
     whether it is the kernel the plain conv would run anyway: the window conv's strided-pixel form (batch one,
@@ -250,7 +256,8 @@ def gn_stats_fits(in_channels: int, out_channels: int, out_d: int, out_h: int, o
     128 or more 512 x 128 output tiles (fewer run as the implicit GEMM, which fills the GPU better)."""
     tiles = out_d * (out_h * out_w // 512) * (out_channels // 128)
     return (batch == 1 and in_channels % 128 == 0 and out_channels in (128, 256) and out_w % 64 == 0
-            and out_w >= 128 and out_d >= 1 and out_h >= 8 and out_h % 8 == 0 and tiles >= 128)
+            and out_w >= 128 and out_d >= 1 and out_h >= 8 and out_h % 8 == 0 and tiles >= 128
+            and _cols_in_range(in_channels, out_channels, out_h, out_w))
 
 
 def gn_workspace_floats(d: int, h: int, w: int) -> int:
@@ -271,7 +278,8 @@ def padded_output_fits(in_channels: int, out_channels: int, out_h: int, out_w: i
     if in_channels % 64 == 0 and out_channels % 128 == 0 and out_w in (32, 64, 128, 256):
         return out_h >= 2 and out_h % (512 // out_w) == 0
     return (batch == 1 and in_channels % 128 == 0 and out_channels % 128 == 0 and out_w >= 128 and out_w % 64 == 0
-            and out_h >= 8 and out_h % 8 == 0 and out_d * (out_h * out_w // 512) * (out_channels // 128) >= 128)
+            and out_h >= 8 and out_h % 8 == 0 and out_d * (out_h * out_w // 512) * (out_channels // 128) >= 128
+            and _cols_in_range(in_channels, out_channels, out_h, out_w))
 
 
 def _conv3d_from_quantized_padded(qx, activation_scale, qweight, weight_scale, *, bias, residual, residual_bias,

@@ -315,3 +315,20 @@ def test_residual_pack_validation(mods):
             validate(bad, bad, b[: bad.shape[1]] if bad.ndim == 5 else b)
     with pytest.raises(ValueError):
         validate(x, x, b[:128])
+
+
+# -- window convolution at other widths: only within its 32-bit offsets -------------------------------------
+
+@pytest.mark.parametrize("h, w, fits", [(480, 640, True), (2360, 2304, True), (2400, 2432, False)])
+def test_window_conv_offers_stay_in_its_offset_range(pkg, h, w, fits):
+    """Three padded 128-channel frames of 2400 x 2432 pass 2 GiB: those run as the implicit GEMM (up to 4 GiB)."""
+    int8 = importlib.import_module(f"{pkg.__name__}.opt.encoder_int8")
+    assert (3 * (h + 2) * (w + 2) * 128 < 2 ** 31) == fits
+    assert int8.gn_stats_fits(128, 128, 1, h, w) == fits
+    assert int8.padded_output_fits(128, 128, h, w, out_d=1) == fits
+
+
+def test_window_conv_offers_need_weights_in_its_offset_range(pkg):
+    int8 = importlib.import_module(f"{pkg.__name__}.opt.encoder_int8")
+    assert int8.padded_output_fits(4864, 16256, 64, 192, out_d=1)
+    assert not int8.padded_output_fits(4864, 16384, 64, 192, out_d=1)
