@@ -505,7 +505,8 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
             } else {
                 const int ri = r / TWP, owr = r - ri * TWP, ow = ow0 + owr;
                 const int wp = pwo + p.pad_left + p.pad_right;
-                // a tile spans 512 / TWP rows: the offset from tile_out stays below 2^31 elements
+                // 32-bit element offsets from tile_out: a tile spans 512 / TWP rows of a frame, below 2^31 elements
+                // at widths up to 256 and, at a run-time width, by cols_conv_fits
                 *reinterpret_cast<u16x8*>(tile_out + (ri * wp + owr) * (int)p.ldo + gcol) = v;
                 const int oh = oh0 + ri;
                 const bool rt = p.pad_top && oh == 1, rb = p.pad_bottom && oh == p.Ho - 2;
@@ -557,7 +558,7 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                 u16x8 gb{};
                 if (p.gn_bias) gb = *reinterpret_cast<const u16x8*>(p.gn_bias + gcol);
                 // tile row r is output row m0 + (r / TILEW) * Wo + r % TILEW: 32-bit element offsets from the
-                // tile's first row (8 rows of a frame of at most 256 channels)
+                // tile's first row (8 rows of a frame, which cols_conv_fits bounds)
                 uint16_t* const tile_out = out + (int64_t)m0 * p.ldo + gcol;
                 lds_barrier();   // the output tile is complete in LDS
                 // all pieces from LDS first (with the residual added), then the stores
@@ -686,8 +687,8 @@ __device__ __forceinline__ void write_tile(const GemmParams& p, AccV (&acc)[BM /
                 p.ldo <= 65536) {
                 // Every column of the tile lies inside N: a thread keeps one 8-column chunk for all its rows,
                 // reads all its pieces from LDS first and stores them from the tile's first output row with
-                // 32-bit element offsets (the tile spans at most 512 consecutive rows, or 8 rows of a frame);
-                // rows past M (the last tile of a GEMM) are skipped.
+                // 32-bit element offsets (the tile spans at most 512 consecutive rows, or 8 rows of a frame, which
+                // cols_conv_fits bounds); rows past M (the last tile of a GEMM) are skipped.
                 constexpr int PER = BM * RCH / NT;
                 const int ch = tid % RCH;
                 uint16_t* const tile_out = out + (int64_t)m0 * p.ldo + gcol0 + ch * 8;
@@ -2328,13 +2329,15 @@ bool halo_conv_fits(const GemmParams& p, int es = 1) {
 }
 
 // Whether a stride-1 3x3x3 convolution with ES-byte elements takes the strided-pixel kernel: whole 8-row tiles of
-// 64-pixel column blocks and stages in groups of four (C * ES % 128 == 0).  Weights of 2 GiB and more, past its
-// 32-bit offsets, stay with the implicit GEMM, which takes up to 4 GiB.
+// 64-pixel column blocks and stages in groups of four (C * ES % 128 == 0).  What passes its signed 32-bit offsets
+// stays with the implicit GEMM, which takes operands of up to 4 GiB and forms its output offsets in 64 bits: three
+// input frames (bytes), the weights (bytes), and the eight rows of a (padded) output frame that a tile stores to
+// (elements: 8 x 300032 outputs of 1024 channels, or 8 x 18752 of 16384).
 bool cols_conv_fits(const GemmParams& p, int es = 1) {
     const bool shape = p.KH == 3 && p.KW == 3 && p.K == 27 * p.C && p.SD == 1 && p.SH == 1 && p.SW == 1 &&
                        (p.C * es) % 128 == 0 && p.N % 128 == 0 && p.Wo % 64 == 0 && p.Ho % 8 == 0;
     return shape && aligned(p.a, 16) && aligned(p.b, 16) && (int64_t)p.Hp * p.Wp * p.C * es * 3 < ((int64_t)1 << 31) &&
-           (int64_t)p.N * p.K * es < ((int64_t)1 << 31);
+           (int64_t)p.N * p.K * es < ((int64_t)1 << 31) && 8 * ((int64_t)p.Wo + 2) * p.N < ((int64_t)1 << 31);
 }
 
 enum class F16Kind { Cols, Halo256, Halo128, Halo64, Halo32, Tiled512x128, Tiled256x128, Tiled256x256, Tiled192x256,
@@ -2810,7 +2813,8 @@ int h3v_conv3d_i8_cols(const int8_t* qx, const float* x_scale, const int8_t* qw,
     p.causal_skip = causal_skip ? 1 : 0;
     H3V_REQUIRE(cols_conv_fits(p) && cout <= 65536 && (padded || cout == 128 || cout == 256),
                 "%s: needs Cin %% 128 == 0, Cout %% 128 == 0 (128 or 256 with statistics), an output width that is a "
-                "multiple of 64 and an output height that is a multiple of 8 (got Cin %d, Cout %d, output %d x %d)", what,
+                "multiple of 64, an output height that is a multiple of 8, and 32-bit offsets that reach three input "
+                "frames, the weights and eight output rows (got Cin %d, Cout %d, output %d x %d)", what,
                 cin, cout, p.Ho, p.Wo);
     H3V_REQUIRE(aligned(out, 16) && (!residual || aligned(residual, 16)) && (!residual_bias || aligned(residual_bias, 16)) &&
                     (!gn_bias || aligned(gn_bias, 16)) && aligned(workspace, 16),

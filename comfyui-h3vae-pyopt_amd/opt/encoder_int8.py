@@ -244,9 +244,11 @@ def _aligned16(t):
 
 
 def _cols_in_range(in_channels: int, out_channels: int, out_h: int, out_w: int) -> bool:
-    """Whether three padded input frames and the weights stay within the window conv's signed 32-bit byte offsets;
-    larger ones (a 2400 x 2432 image at 128 channels) run as the implicit GEMM, which takes up to 4 GiB."""
-    return 3 * (out_h + 2) * (out_w + 2) * in_channels < 2 ** 31 and 27 * in_channels * out_channels < 2 ** 31
+    """Whether a conv stays within the window conv's signed 32-bit offsets: three padded input frames and the weights
+    (bytes), and eight rows of a padded output frame (elements).  Larger ones (a 2400 x 2432 image at 128 channels)
+    run as the implicit GEMM, which takes operands of up to 4 GiB and outputs of any row length."""
+    return (3 * (out_h + 2) * (out_w + 2) * in_channels < 2 ** 31 and 27 * in_channels * out_channels < 2 ** 31
+            and 8 * (out_w + 2) * out_channels < 2 ** 31)
 
 
 def gn_stats_fits(in_channels: int, out_channels: int, out_d: int, out_h: int, out_w: int, *, batch: int = 1) -> bool:

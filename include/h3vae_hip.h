@@ -285,7 +285,9 @@ int h3v_conv3d_i8_gn(const int8_t* qx, const float* x_scale, const int8_t* qw, c
 
 /* The two entries above at any output size of whole 8-row x 64-column tiles
  * (frames encoded untiled): batch one, wo a multiple of 64, ho a multiple of
- * 8, cin % 128 == 0, cout % 128 == 0.  Either padded != 0: the padded output
+ * 8, cin % 128 == 0, cout % 128 == 0, three input frames and the weights
+ * under 2 GiB each, 8 (wo + 2) cout < 2^31 (larger ones are refused; the plain
+ * entry takes them).  Either padded != 0: the padded output
  * of h3v_conv3d_i8_residual_padded (residual, residual_bias, front and the
  * border as there; workspace null), or the statistics of h3v_conv3d_i8_gn
  * (cout 128 or 256; residual, gn_bias and workspace as there; residual_bias

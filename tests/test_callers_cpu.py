@@ -332,3 +332,30 @@ def test_window_conv_offers_need_weights_in_its_offset_range(pkg):
     int8 = importlib.import_module(f"{pkg.__name__}.opt.encoder_int8")
     assert int8.padded_output_fits(4864, 16256, 64, 192, out_d=1)
     assert not int8.padded_output_fits(4864, 16384, 64, 192, out_d=1)
+
+
+# eight output rows: 8 (Wo + 2) Cout < 2^31 elements, with the input frames and the weights in range on both sides
+OUTPUT_RANGE = [(128, 1024, 8, 262080, True), (128, 1024, 8, 262144, False), (128, 1024, 8, 300032, False),
+                (128, 16384, 8, 16320, True), (128, 16384, 8, 18752, False)]
+
+
+@pytest.mark.parametrize("cin, cout, h, w, fits", OUTPUT_RANGE)
+def test_window_conv_offers_need_output_rows_in_its_offset_range(pkg, cin, cout, h, w, fits):
+    int8 = importlib.import_module(f"{pkg.__name__}.opt.encoder_int8")
+    assert 3 * (h + 2) * (w + 2) * cin < 2 ** 31 and 27 * cin * cout < 2 ** 31
+    assert ((7 * (w + 2) + 64) * cout < 2 ** 31) or not fits      # a tile's last store stays in range where it is taken
+    assert int8.padded_output_fits(cin, cout, h, w, out_d=1) == fits
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the accepted shapes would launch on addresses that hold nothing")
+@pytest.mark.parametrize("cin, cout, h, w, fits", OUTPUT_RANGE)
+def test_window_conv_library_rule_matches_the_offers(pkg, cin, cout, h, w, fits):
+    """The rule that all entries share: a shape in its range gets as far as the launch, which fails here without a
+    GPU (RuntimeError), one out of range is refused (ValueError) and left to the implicit GEMM by the plain entries."""
+    hip = importlib.import_module(f"{pkg.__name__}._hip")
+    with pytest.raises(RuntimeError if fits else ValueError, match="LDS|device" if fits else "32-bit offsets"):
+        hip.call("h3v_conv3d_i8_cols", 16, 16, 16, 16, None, None, None, 16, cin, 3, h + 2, w + 2, cout, 1, 1, 2, 0, 1, 0, 1,
+                 None, None, None)
+    # the plain entry takes both; the LDS its launch asks for names the kernel (window 140 KB, implicit GEMM 160 KB)
+    with pytest.raises(RuntimeError, match="143360 bytes" if fits else "163840 bytes"):
+        hip.call("h3v_conv3d_i8", 16, 16, 16, 16, None, 16, 1, cin, 3, h + 2, w + 2, cout, 3, 3, 3, 1, 1, 1, 1, None)
