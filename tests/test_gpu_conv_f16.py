@@ -66,20 +66,47 @@ def _run(fc, x, wt, bias, causal_skip, stride=(1, 1, 1)):
     return y
 
 
-# (batch, Cin, D, H, W, Cout): output widths 32 / 64 / 128 / 256, one and several items, Cin 32..512
+def _run_without_workspace(fc, x, wt, bias, causal_skip, residual=None):
+    """The same stride-1 conv through the entry that takes no workspace, so that nothing splits its reduction."""
+    xd = x.to(DEV).contiguous(memory_format=torch.channels_last_3d)
+    wp = fc.pack_conv_weight_f16(wt.to(DEV))
+    bd = None if bias is None else bias.to(DEV)
+    b, c, d, h, w = x.shape
+    cout, _, kd, kh, kw = wt.shape
+    out = torch.empty((b, cout, d - kd + 1, h - kh + 1, w - kw + 1), dtype=torch.float16, device=DEV,
+                      memory_format=torch.channels_last_3d)
+    fc._hip.call("h3v_conv3d_f16", fc._hip.ptr(xd), fc._hip.ptr(wp), fc._hip.ptr(bd), fc._hip.ptr(residual),
+                 fc._hip.ptr(out), b, c, d, h, w, cout, kd, kh, kw, 1, 1, 1, int(causal_skip), fc._hip.stream(DEV))
+    torch.cuda.synchronize()
+    return out
+
+
+def _splits(fc, b, c, d, h, w, cout, kernel=(3, 3, 3)):
+    """K splits the entry with a workspace takes for a stride-1 conv (0: it does not split)."""
+    kd, kh, kw = kernel
+    outputs = b * (d - kd + 1) * (h - kh + 1) * (w - kw + 1) * cout
+    floats = int(fc._hip.lib().h3v_conv3d_f16_workspace_floats(b, c, d, h, w, cout, *kernel, 1, 1, 1))
+    assert floats % outputs == 0
+    return floats // outputs
+
+
+# (batch, Cin, D, H, W, Cout, bias, K splits with a workspace): output widths 32 / 64 / 128 / 256, one and several
+# items, Cin 32..512; without a workspace all of them run on the window kernel, whole output rows but for the second
 CASES = [
-    (1, 32, 4, 18, 34, 128, True),
-    (3, 256, 5, 10, 66, 128, True),
-    (2, 128, 4, 6, 130, 256, False),
-    (1, 64, 3, 4, 258, 128, True),
-    (4, 512, 3, 18, 34, 256, True),
-    (4, 256, 6, 34, 34, 512, False),
+    (1, 32, 4, 18, 34, 128, True, 0),
+    (3, 256, 5, 10, 66, 128, True, 0),      # column blocks
+    (1, 96, 4, 10, 66, 128, True, 0),
+    (2, 128, 4, 6, 130, 256, False, 6),
+    (1, 64, 3, 4, 258, 128, True, 0),
+    (4, 512, 3, 18, 34, 256, True, 8),
+    (4, 256, 6, 34, 34, 512, False, 0),     # with a workspace: 256 x 128 tiles of the implicit GEMM, unsplit
 ]
 
 
-@pytest.mark.parametrize("b,c,d,h,w,cout,with_bias", CASES)
-def test_conv3d_f16_matches_float64(fc, b, c, d, h, w, cout, with_bias):
+@pytest.mark.parametrize("b,c,d,h,w,cout,with_bias,splits", CASES)
+def test_conv3d_f16_matches_float64(fc, b, c, d, h, w, cout, with_bias, splits):
     print(f"conv3d_f16 B={b} C={c} D={d} {h}x{w} Cout={cout} bias={with_bias}", flush=True)
+    assert _splits(fc, b, c, d, h, w, cout) == splits
     x, wt, bias = _operands(b, c, d, h, w, cout, with_bias, seed=b * 1000 + c + d + h + w + cout)
     y = _run(fc, x, wt, bias, causal_skip=True)
     assert y.shape == (b, cout, d - 2, h - 2, w - 2) and y.dtype == torch.float16
@@ -89,6 +116,9 @@ def test_conv3d_f16_matches_float64(fc, b, c, d, h, w, cout, with_bias):
     # the causal skip drops only taps on zero frames: the full reduction gives the same values
     y_full = _run(fc, x, wt, bias, causal_skip=False)
     assert torch.equal(y_full, y)
+    window = _run_without_workspace(fc, x, wt, bias, causal_skip=True)
+    _assert_close(window, ref, mag)
+    assert torch.equal(_run_without_workspace(fc, x, wt, bias, causal_skip=False), window)
 
 
 def test_conv3d_f16_nonzero_leading_frames_without_skip(fc):
@@ -128,7 +158,7 @@ GEMM_CASES = [
     (3, 256, 4, 8, 8, 512, (1, 1, 1), (1, 1, 1)),          # nin_shortcut
     (1, 128, 3, 20, 20, 200, (3, 3, 3), (1, 1, 1)),
     (1, 96, 4, 12, 12, 256, (3, 3, 3), (1, 1, 1)),          # 64-byte steps on 256 x 128 tiles (few tiles)
-    (1, 256, 3, 18, 18, 1024, (3, 3, 3), (1, 1, 1)),        # 16^2 width, Cout 1024 on 256 x 128 tiles
+    (1, 256, 3, 18, 18, 1024, (3, 3, 3), (1, 1, 1)),        # 16^2 width, Cout 1024: 192-row tiles, 9 splits
 ]
 
 
@@ -146,26 +176,25 @@ def test_conv3d_f16_implicit_gemm_matches_float64(fc, b, c, d, h, w, cout, kerne
     _assert_close(y, ref, mag)
 
 
-# K split over a workspace: (batch, Cin, D, H, W, Cout, causal zero frames, residual); tiles fill under half
-# a round, so S workgroups per tile write fp32 partial sums that a second kernel adds
+# K split over a workspace: (batch, Cin, D, H, W, Cout, causal zero frames, residual, splits); the tiles leave CUs
+# idle, so several workgroups per tile write fp32 partial sums that a second kernel adds
 SPLIT_CASES = [
-    (1, 1024, 7, 18, 18, 48, False, False),     # conv_out-like: Cout 48 on 256 x 128 tiles, 16 splits
-    (1, 256, 7, 18, 18, 256, False, True),      # 256 x 256 tiles, 12 splits, with a residual
-    (2, 256, 5, 18, 18, 256, True, False),      # causal skip: frames 0 / 1 leave whole splits empty
-    (1, 256, 3, 66, 66, 256, True, True),       # one output frame: two of the three depth taps skipped
-    (1, 512, 7, 34, 34, 512, True, False),      # a window-kernel width, split instead
-    (1, 512, 5, 42, 30, 512, True, True),       # 192-row tiles, a last tile across the end
-    (1, 128, 7, 50, 34, 256, False, False),     # window width, K of 54 blocks
+    (1, 1024, 7, 18, 18, 48, False, False, 16),   # conv_out-like: Cout 48 on 256 x 128 tiles
+    (1, 256, 7, 18, 18, 256, False, True, 12),    # 192-row tiles, with a residual
+    (2, 256, 5, 18, 18, 256, True, False, 12),    # causal skip: every split skips the same depth taps of frames 0 / 1
+    (1, 256, 3, 66, 66, 256, True, True, 4),      # one output frame: two of the three depth taps skipped
+    (1, 512, 7, 34, 34, 512, True, False, 4),     # a window-kernel width, split instead
+    (1, 512, 5, 42, 30, 512, True, True, 6),      # 192-row tiles, a last tile across the end
+    (1, 128, 7, 50, 34, 256, False, False, 3),    # window width, K of 54 blocks
 ]
 
 
-@pytest.mark.parametrize("b,c,d,h,w,cout,causal,with_res", SPLIT_CASES)
-def test_conv3d_f16_split_reduction_matches_float64(fc, b, c, d, h, w, cout, causal, with_res):
+@pytest.mark.parametrize("b,c,d,h,w,cout,causal,with_res,splits", SPLIT_CASES)
+def test_conv3d_f16_split_reduction_matches_float64(fc, b, c, d, h, w, cout, causal, with_res, splits):
     print(f"conv3d_f16 split-K B={b} C={c} D={d} {h}x{w} Cout={cout} causal={causal} residual={with_res}", flush=True)
     lib = fc._hip.lib()
     floats = int(lib.h3v_conv3d_f16_workspace_floats(b, c, d, h, w, cout, 3, 3, 3, 1, 1, 1))
-    m = b * (d - 2) * (h - 2) * (w - 2)
-    assert floats > 0 and floats % (m * cout) == 0 and floats // (m * cout) >= 2   # the geometry splits
+    assert _splits(fc, b, c, d, h, w, cout) == splits
     x, wt, bias = _operands(b, c, d, h, w, cout, True, seed=c + cout + d, causal_zero=causal)
     gen = torch.Generator().manual_seed(cout)
     res = (torch.randn(b, cout, d - 2, h - 2, w - 2, generator=gen) * 2).half() if with_res else None
@@ -192,6 +221,45 @@ def test_conv3d_f16_split_reduction_matches_float64(fc, b, c, d, h, w, cout, cau
         fc._hip.call("h3v_conv3d_f16_ws", fc._hip.ptr(xd), fc._hip.ptr(wp), fc._hip.ptr(bias.to(DEV)), None,
                      fc._hip.ptr(out), b, c, d, h, w, cout, 3, 3, 3, 1, 1, 1, int(causal), fc._hip.ptr(ws),
                      floats - 1, fc._hip.stream(DEV))
+
+
+# The ping-pong convolution (Cout > 128, channel bytes a multiple of 128) in its other forms: (batch, Cin, D, H, W,
+# Cout, kernel, splits).  1x1x1 kernels run one, two and three K steps (the schedule's prologue alone, and with one
+# step past it), the 3x3x3 ones 27 with causal depth taps skipped in tiles that span two items.  Unsplit: 251 tiles
+# of 192 rows, or 254 of 256 where the 192-row ones would need a second round; both end in a tile that M cuts, and
+# Cout 200 in columns that it cuts.
+WIDE_CASES = [
+    (1, 64, 5, 97, 99, 200, (1, 1, 1), 0), (1, 128, 5, 97, 99, 200, (1, 1, 1), 0), (1, 192, 5, 97, 99, 200, (1, 1, 1), 0),
+    (2, 64, 5, 91, 92, 256, (3, 3, 3), 0),
+    (1, 64, 5, 113, 115, 200, (1, 1, 1), 0), (1, 128, 5, 113, 115, 200, (1, 1, 1), 0),
+    (1, 192, 5, 113, 115, 200, (1, 1, 1), 0), (2, 64, 5, 106, 106, 256, (3, 3, 3), 0),
+    (1, 256, 4, 47, 47, 1000, (3, 3, 3), 4),       # 64 tiles of 256 rows four ways (86 of 192 rows would fit twice)
+    (1, 2048, 5, 6, 7, 132, (3, 1, 1), 12),        # 32 blocks a depth tap in shares of 3: the last split has none
+]
+
+
+@pytest.mark.parametrize("b,c,d,h,w,cout,kernel,splits", WIDE_CASES)
+def test_conv3d_f16_pingpong_tiles_match_float64(fc, b, c, d, h, w, cout, kernel, splits):
+    print(f"conv3d_f16 ping-pong B={b} C={c} D={d} {h}x{w} Cout={cout} k={kernel}", flush=True)
+    assert _splits(fc, b, c, d, h, w, cout, kernel) == splits
+    causal = kernel[0] == 3
+    gen = torch.Generator().manual_seed(c + d + h + w + cout)
+    x = torch.randn(b, c, d, h, w, generator=gen).half()
+    if causal:
+        x[:, :, :2] = 0
+    wt = (torch.randn(cout, c, *kernel, generator=gen) * (c * kernel[0] * kernel[1] * kernel[2]) ** -0.5).half()
+    bias = (0.5 * torch.randn(cout, generator=gen)).half()
+    xd, wp, bd = x.to(DEV).contiguous(memory_format=torch.channels_last_3d), fc.pack_conv_weight_f16(wt.to(DEV)), bias.to(DEV)
+    with torch.inference_mode():
+        y = fc.conv3d_f16(xd, wp, bd, list(kernel), [1, 1, 1], causal)
+        res = torch.randn(y.shape, generator=gen).half().to(DEV).contiguous(memory_format=torch.channels_last_3d)
+        fused = fc.conv3d_f16(xd, wp, bd, list(kernel), [1, 1, 1], causal, res)
+        torch.cuda.synchronize()
+    assert torch.equal(fused, res + y)
+    for t in range(y.shape[2]):                      # every output frame from its own input frames
+        xs = x[:, :, t:t + kernel[0]].double()
+        ref, mag = F.conv3d(xs, wt.double(), bias.double()), F.conv3d(xs.abs(), wt.double().abs())
+        _assert_close(y[:, :, t:t + 1], ref, mag)
 
 
 @pytest.mark.parametrize("c,d,h,w", [(512, 7, 34, 34), (512, 5, 42, 30)])
