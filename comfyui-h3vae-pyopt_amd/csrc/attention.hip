@@ -459,7 +459,8 @@ AttnPlan plan_attention(int64_t batch, int64_t tokens, int64_t heads, bool may_s
     const int64_t rounds = t / kCUs, full = rounds * kCUs / bh;   // 512-query blocks per head in whole rounds
     const int64_t rest = tokens - 512 * full, w = (rest + 255) / 256 * bh;
     if (full > 0 && 16 * full * bh >= 15 * rounds * kCUs && w <= 128) {
-        // at least 4 key blocks a split (tokens > 512 here, so a split always has some)
+        // split sizes of at least 4 key blocks (tokens > 512 here); they are rounded up, so the last split may be
+        // shorter, down to one block
         int64_t splits = may_split ? kCUs / w : 1;
         splits = splits < nblk / 4 ? splits : nblk / 4;
         splits = splits < 1 ? 1 : (splits > 16 ? 16 : splits);
