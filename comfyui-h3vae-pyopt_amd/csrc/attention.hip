@@ -445,10 +445,15 @@ struct AttnPlan {
 //   t <= 256         512 queries            2 x 1797: 75.0 / 87.9 / 85.2 / 92.7
 // Beyond one round, workgroups of 512 for the whole rounds; the queries past them, when they are at most 128
 // workgroups of 256 queries and the full rounds are nearly full, run with their keys split so that they fill the
-// chip too (1 x 8405: 825.6 -> 651.7; 1 x 4100: 277.3 -> 179.1; error against 64 bits unchanged, 2.96e-4).  Otherwise 4-wave workgroups, two of which share a
-// CU, where the last round is under 3/4 full (3 x 1797: 133.5 / 128.8 / 125.7 / 130.7; 1 x 7173, 15/16 full:
-// 495.2 / 587.7 / 559.3 / 620.6).
-AttnPlan plan_attention(int64_t batch, int64_t tokens, int64_t heads, bool may_split) {
+// chip too (1 x 8405: 825.6 -> 651.7; 1 x 4100: 277.3 -> 179.1; error against 64 bits unchanged, 2.96e-4).
+// Otherwise 4-wave workgroups, two of which share a CU, where the last round is at most half full, so that its
+// workgroups of 256 queries find a CU each, in a call of under four rounds (or of rows so short that the rounds stay
+// together): 512 against 256 on 4 waves, 3 x 1797 135.7 / 125.7, 1 x 6144 412.7 / 388.3, 1 x 10240 1046.5 / 1027.0,
+// 1 x 14336 1992.9 / 1981.4, 33 x 453 125.2 / 114.2.  With the last round 5/8 full a CU gets two of them
+// (1 x 6200 412.3 / 470.0, 1 x 10400 1063.4 / 1198.6), in more rounds their ends drift apart (2 x 11205 2320 / 2443,
+// 13 x 1797 498.5 / 515.1), and beside another stream's call their smaller share of each key block counts: decoding
+// with 3 x 1797 or 2 x 2805 tokens on two tile streams took 2% longer with them.
+AttnPlan plan_attention(int64_t batch, int64_t tokens, int64_t heads, bool may_split, bool on_its_own) {
     constexpr int64_t kCUs = 256;
     const int64_t bh = batch * heads, nblk = (tokens + kBK - 1) / kBK;
     const int64_t t = (tokens + 511) / 512 * bh;
@@ -469,7 +474,7 @@ AttnPlan plan_attention(int64_t batch, int64_t tokens, int64_t heads, bool may_s
         plan.splits = (int)((nblk + plan.split_blocks - 1) / plan.split_blocks);
         return plan;
     }
-    if (4 * (t - rounds * kCUs) < 3 * kCUs) plan.shape = AttnShape::Q256x4;
+    if (on_its_own && 2 * (t - rounds * kCUs) <= kCUs && (rounds < 4 || tokens <= 1024)) plan.shape = AttnShape::Q256x4;
     return plan;
 }
 
@@ -513,7 +518,7 @@ static int attention_common(const char* what, const uint16_t* q, int64_t q_token
     p.o_ts = o_token_stride; p.o_hs = o_head_stride;
     p.tokens = (int)tokens;
     p.c = scale * 1.4426950408889634f;
-    const AttnPlan plan = plan_attention(batch, tokens, heads, may_split);
+    const AttnPlan plan = plan_attention(batch, tokens, heads, may_split, alone(stream));
     const int64_t floats = attention_ws_floats(plan, batch, tokens, heads);
     H3V_REQUIRE(floats == 0 || (workspace && workspace_floats >= floats && aligned(workspace, 16)),
                 "%s: needs a 16-byte aligned workspace of %lld floats", what, (long long)floats);
@@ -556,7 +561,8 @@ extern "C" int h3v_attention_d64(const uint16_t* q, int64_t q_token_stride, int6
 
 extern "C" int64_t h3v_attention_d64_workspace_floats(int64_t batch, int64_t tokens, int64_t heads) {
     if (batch <= 0 || tokens <= 0 || heads <= 0 || batch > 65535 || heads > 65535 || tokens > (1 << 24)) return 0;
-    return attention_ws_floats(plan_attention(batch, tokens, heads, true), batch, tokens, heads);
+    // a split does not depend on the stream
+    return attention_ws_floats(plan_attention(batch, tokens, heads, true, true), batch, tokens, heads);
 }
 
 extern "C" int h3v_attention_d64_ws(const uint16_t* q, int64_t q_token_stride, int64_t q_head_stride, const uint16_t* k,

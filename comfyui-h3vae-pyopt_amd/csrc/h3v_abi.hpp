@@ -20,6 +20,12 @@ int launch_status(const char* what);
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
+// Whether a launch on this stream is taken to have the chip to itself.  Programs that overlap independent work (the
+// package's tile streams, two decoder calls at a time) put it on streams of their own, where a plan that spends more
+// of the chip to end its own call sooner takes that time from the other call: such plans are for the default stream.
+// The results do not depend on it.
+inline bool alone(hipStream_t stream) { return stream == nullptr; }
+
 }  // namespace h3v
 
 #define H3V_REQUIRE(cond, ...)                                   \

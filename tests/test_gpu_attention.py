@@ -161,6 +161,22 @@ def test_attention_workgroup_shapes_and_key_splits(ops, oracle, b, n, h, head):
     assert float((out.float() - plain.float()).abs().max()) < 2e-3
 
 
+# last rounds of 512-query workgroups half full, 5/8 full, and after four rounds; a key split
+@pytest.mark.parametrize("b,n,h", [(12, 453, 32), (13, 453, 32), (33, 453, 32), (2, 2049, 32)])
+def test_attention_on_another_stream(ops, b, n, h):
+    """A call on another stream than the default one may take larger workgroups; every query keeps its wave's 64."""
+    print(f"attention on another stream [{b}, {n}, {h}, 64]", flush=True)
+    _, _, _, qd, kd, vd = _qkv(b, n, h, seed=b + n)
+    att, side = ops.decoder_fused_qk_rope.attention_d64, torch.cuda.Stream()
+    with torch.inference_mode():
+        out = att(qd, kd, vd, 0.125)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            other = att(qd, kd, vd, 0.125)
+        torch.cuda.synchronize()
+    assert torch.equal(other, out)
+
+
 @pytest.mark.parametrize("ramp", [False, True])
 @pytest.mark.parametrize("b", [4, 8, 10])    # 256 queries per workgroup, 512, 256 on four waves; one item alone: 128
 def test_attention_of_an_item_alone_and_in_a_batch(ops, b, ramp):

@@ -45,7 +45,9 @@ def _oracle(oracle, x, gamma, beta, pb, b, eps):
                                           (1024, 1, 2, 3, 29, True), (1024, 1, 2, 2, 30, False),
                                           (1024, 1, 1, 5, 31, True), (512, 1, 2, 3, 62, False),
                                           (256, 1, 3, 4, 127, True), (128, 1, 1, 4, 190, False),
-                                          (256, 2, 7, 300, 6, True)])
+                                          (256, 2, 7, 300, 6, True),
+                                          # 20 chunks a frame, the most that the pack merges itself, and 21
+                                          (1024, 1, 1, 32, 40, True), (1024, 1, 1, 21, 61, False)])
 def test_norm_pack_f16_matches_oracle(ops, oracle, c, b, d, h, w, pb):
     print(f"norm_pack_f16 C={c} B={b} D={d} {h}x{w} pre_bias={pb}", flush=True)
     x, gamma, beta, pre = _inputs(b, c, d, h, w, pb, seed=c + b + d + h + w)
