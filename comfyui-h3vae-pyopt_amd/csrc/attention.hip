@@ -93,7 +93,8 @@ __global__ __launch_bounds__(64 * NW) void fmha_d64(AttnParams p) {
     const int h = blockIdx.y, b = PART ? blockIdx.z / p.splits : blockIdx.z;
     const int n = p.tokens;
     const int64_t row0 = (int64_t)b * n;                 // first token row of this batch item
-    const int q0 = p.q_first + blockIdx.x * BQ + wave * 32 * QS;   // the wave's first query
+    // the wave's first query; only the one-set workgroups run the queries past others
+    const int q0 = (QS == 1 ? p.q_first : 0) + blockIdx.x * BQ + wave * 32 * QS;
     const int hi = lane >> 5;                           // which 8 of a 16-wide k chunk this lane holds
     const bool wave_active = q0 < n;                    // wave-uniform
 
