@@ -2564,11 +2564,15 @@ enum class SmallTile { None, T64, T128, T128x2 };
 //   then up to 512 with a two-stage ring, so    3594 x 2048 x 8192: 96.5 / 68.5 / 62.8 / 76.1;
 //   that two workgroups share a CU              453 x 16384 x 2048: 32.6 / 27.5 / 22.4 / 27.2;
 //   beyond                                      4100 x 2048 x 2048: 35.1 / 36.2 / 33.0 / 28.0.
-SmallTile small_tile(int64_t m, int64_t n) {
+// The tiles two per CU end a call sooner but read their operands twice as often as the ping-pong tiles; beside another
+// stream's call, which uses the CUs that those leave, they cost more than they save.  A six-block decoder on 7 x 48 x 84
+// latents, with them (and the rows past the last round on 128 x 128 tiles, below) against without: on two tile streams
+// 37.2 / 35.5 ms at 3594 rows a call and 40.7 / 39.0 at 4052, on one stream 40.2 / 41.4 and 43.8 / 44.9.
+SmallTile small_tile(int64_t m, int64_t n, bool on_its_own) {
     auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
     if (tiles(64) <= 512) return SmallTile::T64;
     if (tiles(128) <= 256) return SmallTile::T128;
-    if (tiles(128) <= 512) return SmallTile::T128x2;
+    if (on_its_own && tiles(128) <= 512) return SmallTile::T128x2;
     return SmallTile::None;
 }
 
@@ -2584,17 +2588,19 @@ int launch_small_tile(SmallTile t, const GemmParams& p, hipStream_t stream, cons
 // as a second launch on the remaining rows: 8405 x 2048 x 8192 (264 ping-pong tiles) 171.8 -> 128.3 us, 8405 x
 // 2048 x 2048 55.0 -> 44.4, 3000 x 6144 x 2048 54.7 -> 47.6, 7188 x 16384 x 2048 (7.25 rounds) 250.4 -> 242.4.
 // After three rounds the tiles' ends are spread out and a larger rest overlaps them (8405 x 16384 x 2048, 256
-// tiles of 128 x 128 left after 8 rounds: 288.6 against 301.0 us split), so there only the 64 x 64 tiles split off.
+// tiles of 128 x 128 left after 8 rounds: 288.6 against 301.0 us split), so there only the 64 x 64 tiles split off, as
+// beside another stream's call at any size (3594 rows a call on two tile streams, QKV split or not: 37.2 / 36.0 ms).
 template <Epi EP>
 int run_gemm_k128(const GemmParams& p, hipStream_t stream, const char* what) {
-    const SmallTile whole = small_tile(p.M, p.N);
+    const bool on_its_own = alone(stream);
+    const SmallTile whole = small_tile(p.M, p.N, on_its_own);
     if (whole != SmallTile::None) return launch_small_tile<EP>(whole, p, stream, what);
     const int64_t tn = (p.N + 255) / 256, tiles = (p.M + 255) / 256 * tn;
     const int64_t head = 256 * (tiles / 256 * 256 / tn);   // rows of the full rounds
     const bool in_range = (int64_t)p.M * p.lda < ((int64_t)1 << 32) && (int64_t)p.N * p.K < ((int64_t)1 << 32);
     if (head > 0 && head < p.M && in_range) {
-        const SmallTile rest = small_tile(p.M - head, p.N);
-        if (rest == SmallTile::T64 || (rest != SmallTile::None && tiles < 3 * 256)) {
+        const SmallTile rest = small_tile(p.M - head, p.N, on_its_own);
+        if (rest == SmallTile::T64 || (rest != SmallTile::None && on_its_own && tiles < 3 * 256)) {
             GemmParams h = p, t = p;
             h.M = (int)head;
             t.M = (int)(p.M - head);

@@ -42,8 +42,11 @@ def test_gemm_tiles_exact(oracle, m, n, k, with_bias):
     hip.call("h3v_gemm_i8_i32", hip.ptr(a), hip.ptr(w), hip.ptr(acc), m, n, k, hip.stream(DEV))
     hip.call("h3v_gemm_i8_dequant", hip.ptr(a), hip.ptr(sx), hip.ptr(w), hip.ptr(sw), hip.ptr(bias), hip.ptr(out),
              m, n, k, hip.stream(DEV))
+    side, other = torch.cuda.Stream(), torch.full_like(acc, 7)   # on another stream the choice of tiles is narrower
+    side.wait_stream(torch.cuda.current_stream())
+    hip.call("h3v_gemm_i8_i32", hip.ptr(a), hip.ptr(w), hip.ptr(other), m, n, k, side.cuda_stream)
     torch.cuda.synchronize()
     want = (a.double() @ w.double().t()).to(torch.int32)
-    assert torch.equal(acc, want)
+    assert torch.equal(acc, want) and torch.equal(other, want)
     assert_bitwise(np_(out), oracle.gemm_dequant(np_(want), np_(sx), np_(sw), None if bias is None else np_(bias)), "out")
     assert np.isfinite(np_(out)).all()
