@@ -719,7 +719,8 @@ def cpu_baseline(budget_s: float):
 TRAFFIC_PROFILE = ROOT / "profiles" / "stage0_conv_traffic_pmc.md"
 GEMM_TRAFFIC_PROFILE = ROOT / "profiles" / "int8_gemm_decoder_traffic_pmc.md"
 GEMM_KERNEL = ("gemm_i8_pingpong<Dequant> (every decoder INT8 GEMM: QKV, attention-out and FFN-up with K = 2048, "
-               "FFN-down with K = 8192; 256x256x128 tiles, two wave groups alternating MFMA and fragment-read phases)")
+               "FFN-down with K = 8192; 256x256x128 tiles, two wave groups alternating MFMA and fragment-read phases; "
+               "with FFN-up's rows past the last full round of tiles, a second launch of gemm_i8_small)")
 
 
 def _profile_number(path, key):
