@@ -71,7 +71,7 @@ struct GemmParams {
     int conv_tpf;      // conv: M tiles per output frame when they do not straddle frames, else 0
     uint32_t a_bytes;  // extents of A and W in bytes (buffer resource ranges, < 4 GiB)
     uint32_t b_bytes;
-    int k_splits;      // tiled kernels: K blocks split evenly over gridDim.y = k_splits workgroups (0 or 1: none)
+    int k_splits;      // tiled kernels: K blocks shared by gridDim.y = k_splits workgroups, see k_range (0 or 1: none)
     // statistics epilogue of the window conv (h3v_conv3d_i8_gn; null gn_avg: off): the GroupNorm(32)
     // partial statistics of each 512-pixel output tile, in the producer workspace layout (GnWorkspace)
     float* gn_avg;
@@ -2360,7 +2360,8 @@ int f16_splits(int64_t tiles, int kblocks) {
 
 // Tile and K split of the fp16 implicit GEMM for N > 128, by an estimate in us of the candidates: 256 x 256 and
 // 192 x 256 tiles, unsplit or with a reduction split of at most one round of the CUs that divides the K blocks and
-// leaves each split at least 8 of them, and unsplit 256 x 128 tiles.  A 256 x 256 tile takes about 1.45 us per
+// leaves a split 8 of them on average, and unsplit 256 x 128 tiles (k_range shares out each depth tap, rounded up, so a
+// divisor of all K blocks that does not divide a tap's leaves the last split fewer, or none).  A 256 x 256 tile takes about 1.45 us per
 // block of 128 bytes of K and 8 us around them on a full chip; a 192-row one 3/4 of that and 4% (three instead of
 // four 32-row blocks share a weight fragment), a 256 x 128 one half and 15%; a split's partial sums are written and
 // read at about 5 TB/s, and the second kernel takes 6 us.  Up to three rounds count whole; over more, the tiles'
