@@ -2358,17 +2358,17 @@ int f16_splits(int64_t tiles, int kblocks) {
     return best;
 }
 
-// Tile and K split of the fp16 implicit GEMM for N > 128, by an estimate in us of the candidates: 256 x 256 and
-// 192 x 256 tiles, unsplit or with a reduction split of at most one round of the CUs that divides the K blocks and
-// leaves a split 8 of them on average, and unsplit 256 x 128 tiles (k_range shares out each depth tap, rounded up, so a
-// divisor of all K blocks that does not divide a tap's leaves the last split fewer, or none).  A 256 x 256 tile takes about 1.45 us per
-// block of 128 bytes of K and 8 us around them on a full chip; a 192-row one 3/4 of that and 4% (three instead of
-// four 32-row blocks share a weight fragment), a 256 x 128 one half and 15%; a split's partial sums are written and
-// read at about 5 TB/s, and the second kernel takes 6 us.  Up to three rounds count whole; over more, the tiles'
-// ends drift apart.  `active` is the share of K a tile runs (a causal conv of one frame skips two thirds).
-// Before and now (us, causal): 4 x 512 -> 512 at 5 x 32 x 32 (160 window tiles against 214 of 192 rows) 238.9 ->
-// 225.8, one clip (40 window tiles, six splits) 213.4 -> 78.6, 512 -> 512 at 5 x 60 x 80 (188 tiles of 256 rows,
-// 250 of 192) 284.8 -> 244.2, 512 -> 512 at 1 x 32 x 32 73.8 -> 25.0.
+// Tile and K split of the fp16 implicit GEMM for N > 128, by an estimate in us of the candidates: 256 x 256 and 192 x
+// 256 tiles, unsplit or with a reduction split of at most one round of the CUs that divides the K blocks and leaves a
+// split 8 of them on average, and unsplit 256 x 128 tiles (k_range shares out each depth tap, rounded up, so a divisor
+// of all K blocks that does not divide a tap's leaves the last split fewer, or none).  A 256 x 256 tile takes about
+// 1.45 us per block of 128 bytes of K and 8 us around them on a full chip; a 192-row one 3/4 of that and 4% (three
+// instead of four 32-row blocks share a weight fragment), a 256 x 128 one half and 15%; a split's partial sums are
+// written and read at about 5 TB/s, and the second kernel takes 6 us.  Up to three rounds count whole; over more, the
+// tiles' ends drift apart.  `active` is the share of K a tile runs (a causal conv of one frame skips two thirds).
+// Before and now (us, causal): 4 x 512 -> 512 at 5 x 32 x 32 (160 window tiles against 214 of 192 rows) 238.9 -> 225.8,
+// one clip (40 window tiles, six splits) 213.4 -> 78.6, 512 -> 512 at 5 x 60 x 80 (188 tiles of 256 rows, 250 of 192)
+// 284.8 -> 244.2, 512 -> 512 at 1 x 32 x 32 73.8 -> 25.0.
 struct WidePlan {
     F16Plan plan;
     double us;
